@@ -3,7 +3,10 @@
 // m = 1 with k = 2048 or 4096 (plain layouts): the decode strip kernel, wavefront per N-strip
 // with v_dot8_u32_u4 and DPP / lane-swap reductions (described above w4a8_strip_kernel).
 //
-// Fast path (decode-shaped, any m in chunks of 15 rows, k % 256 == 0): one workgroup of 8
+// Many rows, or k not a multiple of 256 (plain layouts, k % 32 == 0): the large-tile kernel of
+// int8_tile.hpp, which reads the weights once per tile of rows instead of once per 15 rows.
+//
+// Few rows (any m in chunks of 15 rows, k % 256 == 0): one workgroup of 8
 // wave64s owns a 16-channel weight tile (16 rows of B) for one chunk of up to 15 activation
 // rows; wave w owns one eighth of k.
 //   * Plain weights stream in 128-bit loads shaped 8 rows x 128 bytes per wave instruction
@@ -29,6 +32,7 @@
 // correction, two scale multiplies, C, bias, clamp; no FMA) runs per output.
 #include <cfloat>
 
+#include "int8_tile.hpp"
 #include "tqt_hip_common.hpp"
 #include "tqt_gemm_1xnbias_clamp_f32_qai8dx_qsi4cxt_mfma_gfx950.h"
 #include "tqt_gemm_1xnbias_clamp_f32_qai8dxp_qsi4cxp_mfma_gfx950.h"
@@ -66,30 +70,6 @@ struct W4A8Args
     const float *scale_b;
     PackDesc pa, pb;  // packed A / B of the p-variant (read when the kernel's PK bit is set)
 };
-
-// reference tqt_kernel_gemm_i8_i4_4x1vl_rvv.h:234-419: zp correction (int32), RNE convert, two
-// separate multiplies, C then bias (separate adds), vfmax then vfmin.
-__device__ __forceinline__ float epilogue_f32(int32_t acc, int32_t rsum, int32_t zp, float sa,
-                                              float sb, const float *c, const float *bias,
-                                              float cmin, float cmax)
-{
-    // Rounds after every operation: the library is built with -ffp-contract=off, since hipcc
-    // would otherwise fuse a * b + c (__fmul_rn / __fadd_rn do not prevent it).
-    const int32_t v = static_cast<int32_t>(static_cast<uint32_t>(acc) -
-                                           static_cast<uint32_t>(zp) * static_cast<uint32_t>(rsum));
-    float f = __int2float_rn(v);
-    f = __fmul_rn(f, sa);
-    f = __fmul_rn(f, sb);
-    if (c) {
-        f = __fadd_rn(f, *c);
-    }
-    if (bias) {
-        f = __fadd_rn(f, *bias);
-    }
-    f = fmaxf(f, cmin);
-    f = fminf(f, cmax);
-    return f;
-}
 
 // 16 activation bytes -> the byte order of the decoded weights within each 8-byte group:
 // (even k of bytes 0-7, odd k of bytes 0-7, even k of bytes 8-15, odd k of bytes 8-15).
@@ -169,7 +149,7 @@ __global__ __launch_bounds__(kWaves * 64) void w4a8_mfma_kernel(W4A8Args a)
     const int orow = tid >> 4;
     const int ocol = tid & 15;
     const bool out_ok = tid < 256 && orow < rows && n0 + ocol < a.N;
-    float p_sb = 0.f, p_sa = 0.f, p_bias = 0.f, p_c = 0.f;
+    float p_sb = 0.f, p_sa = 0.f, p_bias = -0.f, p_c = -0.f;
     int32_t p_za = 0;
     // output rows are addressed as the workgroup's first row (uniform, 64-bit) plus a 24-bit
     // per-thread offset (the launcher keeps ldc, ldd, lda and the weight row stride < 2^24)
@@ -388,9 +368,8 @@ __global__ __launch_bounds__(kWaves * 64) void w4a8_mfma_kernel(W4A8Args a)
         const int gn = n0 + ocol;
         store_out<OUT>(a.D, static_cast<long long>(m0) * a.ldd +
                                 __umul24(orow, static_cast<uint32_t>(a.ldd)) + gn,
-                       epilogue_f32(static_cast<int32_t>(tot) >> 4, static_cast<int32_t>(rs) >> 4,
-                                    p_za, p_sa, p_sb, a.C ? &p_c : nullptr,
-                                    a.bias ? &p_bias : nullptr, a.cmin, a.cmax));
+                       w4a8_value(static_cast<int32_t>(tot) >> 4, static_cast<int32_t>(rs) >> 4, p_za,
+                                  p_sa, p_sb, p_c, p_bias, a.cmin, a.cmax));
     }
 }
 
@@ -551,9 +530,8 @@ __device__ __forceinline__ void strip_finish(const W4A8Args &a, int n0, int lane
     const int oc = lane >> 4;
     if ((lane & 15) == 0 && n0 + oc < a.N) {
         store_out<OUT>(a.D, n0 + oc,
-                       epilogue_f32(static_cast<int32_t>(tot), 0, 0, p_sa, p_sb,
-                                    a.C ? &p_c : nullptr, a.bias ? &p_bias : nullptr, a.cmin,
-                                    a.cmax));
+                       w4a8_value(static_cast<int32_t>(tot), 0, 0, p_sa, p_sb, p_c, p_bias, a.cmin,
+                                  a.cmax));
     }
 }
 
@@ -609,8 +587,8 @@ __global__ __launch_bounds__(kStripWaves * 64) void w4a8_strip_kernel(W4A8Args a
     const int gn = min(n0 + (lane >> 4), a.N - 1);
     const float p_sb = a.scale_b[gn];
     const float p_sa = a.scale_a[0];
-    const float p_bias = a.bias ? load_out<OUT>(a.bias, gn) : 0.f;
-    const float p_c = a.C ? load_out<OUT>(a.C, gn) : 0.f;
+    const float p_bias = a.bias ? load_out<OUT>(a.bias, gn) : -0.f;
+    const float p_c = a.C ? load_out<OUT>(a.C, gn) : -0.f;
     strip_finish<L, OUT>(a, n0, lane, av, wv, zp, p_sa, p_sb, p_bias, p_c);
 }
 
@@ -658,8 +636,8 @@ __global__ __launch_bounds__(kStripWaves * 64) void w4a8_qstrip_kernel(W4A8Args 
     asm volatile("" ::: "memory");
     const int gn = min(n0 + (lane >> 4), a.N - 1);
     const float p_sb = a.scale_b[gn];
-    const float p_bias = a.bias ? load_out<OUT>(a.bias, gn) : 0.f;
-    const float p_c = a.C ? load_out<OUT>(a.C, gn) : 0.f;
+    const float p_bias = a.bias ? load_out<OUT>(a.bias, gn) : -0.f;
+    const float p_c = a.C ? load_out<OUT>(a.C, gn) : -0.f;
 
     // the row's minimum and maximum (exact: any order)
     float lo = FLT_MAX, hi = -FLT_MAX;
@@ -761,6 +739,100 @@ bool launch_w4a8_qstrip(const W4A8Args &a, const float *X, int8_t *Aq, float *sa
     return true;
 }
 
+// ---------------------------------------------------------------------------------------------
+// Large-tile kernel (int8_tile.hpp): which tile a shape takes. Every tile is one pass of a CU over
+// k, so the launch costs ceil(tiles / 256) times (fixed + stages * rate) of its tile; the rates
+// below are microseconds measured on MI355X at k 864 and 4096 (M x N tiles: 256 x 256 82 us for
+// one round of 256 at k 4096, 128 x 128 23, 64 x 128 14.7, 32 x 128 11.7), and the cheapest wins:
+// 1000 x 11008 x 4096 takes 128 x 128 tiles (69 us; 74 with 256 x 256, 79 with 64 x 128, 108 with
+// 32 x 128), 512 x 4096 x 4096 64 x 128 (18.3; 25.7, 21.6 with 32 x 128), 4096^3 256 x 256 (82; 97).
+// The k-split kernel above, where it applies, costs one pass over the weights per 15 rows instead:
+// 3.2 us + 0.115 us per 10^6 weights and pass (11008 x 4096: 8.1 us at 12 rows, 12.6 at 16, 18.5 at
+// 32, 23.0 at 48, against 12.2-12.8 for the tiles; 4096 x 4096: 9.7 at 48 and 27.1 at 200, against
+// 12.5 and 12.8).
+// ---------------------------------------------------------------------------------------------
+constexpr int kTileCUs = 256;  // compute units of an MI355X
+
+struct TileShape
+{
+    int bm, bn;
+    float fixed, stage;  // us per round: fixed + stage * ceil(k / 128)
+};
+constexpr TileShape kTileShapes[] = {
+    {256, 256, 18.0f, 2.0f}, {128, 128, 5.0f, 0.57f}, {64, 128, 4.5f, 0.32f}, {32, 128, 4.0f, 0.24f}};
+
+template <int MI, int NI, int WGM, int WGN, int KS, int NS, int OUT>
+void launch_tile(TileArgs t, hipStream_t s)
+{
+    constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN;
+    t.tiles_m = (t.M + BM - 1) / BM;
+    t.tiles_n = (t.N + BN - 1) / BN;
+    const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;
+    TQT_REQUIRE(tiles < (1ll << 28), "grid too large");
+    t.per_xcd = static_cast<int>((tiles + 7) / 8);
+    hipLaunchKernelGGL((w4a8_tile_kernel<MI, NI, WGM, WGN, KS, NS, OUT>),
+                       dim3(8 * static_cast<unsigned>(t.per_xcd)), dim3(64 * WGM * WGN * KS), 0, s, t);
+}
+
+// The tile kernel for plain layouts whose rows are whole 32-k groups of aligned bytes; false when
+// it does not apply (the kernel's offsets are 32 bits from a tile's first row) or the k-split
+// kernel, if it does (`ksplit`), is the faster one.
+template <int OUT>
+bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
+{
+    if (a.K % 32 != 0 || a.K == 0 || a.K > 65536 || a.lda % 16 != 0 ||
+        a.bstride % 16 != 0 || !aligned16(a.A) || !aligned16(a.B) || a.lda >= (1 << 22) ||
+        a.bstride >= (1 << 22)) {
+        return false;
+    }
+    TileArgs t = {};
+    t.M = a.M;
+    t.N = a.N;
+    t.K = a.K;
+    t.A = a.A;
+    t.lda = a.lda;
+    t.B = a.B;
+    t.bstride = a.bstride;
+    t.C = a.C;
+    t.ldc = a.ldc;
+    t.D = a.D;
+    t.ldd = a.ldd;
+    t.bias = a.bias;
+    t.cmin = a.cmin;
+    t.cmax = a.cmax;
+    t.scale_a = a.scale_a;
+    t.zp_a = a.zp_a;
+    t.scale_b = a.scale_b;
+    constexpr int kElem = OUT == OUT_F32 ? 4 : 2;
+    t.vec_d = a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.D) % (4 * kElem) == 0;
+    const float stages = static_cast<float>((a.K + kTileK - 1) / kTileK);
+    int best = 0;
+    float best_us = 0.f;
+    for (int i = 0; i < 4; ++i) {
+        const TileShape &p = kTileShapes[i];
+        const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
+                                ((a.N + p.bn - 1) / p.bn);
+        const float us = static_cast<float>((tiles + kTileCUs - 1) / kTileCUs) *
+                         (p.fixed + p.stage * stages);
+        if (i == 0 || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    const int passes = (a.M + kRowsPerChunk - 1) / kRowsPerChunk;
+    if (ksplit && 3.2f + 0.115e-6f * static_cast<float>(a.N) * static_cast<float>(a.K) *
+                              static_cast<float>(passes) <= best_us) {
+        return false;
+    }
+    switch (best) {
+    case 0: launch_tile<4, 2, 2, 4, 1, 3, OUT>(t, s); break;
+    case 1: launch_tile<4, 2, 1, 2, 2, 3, OUT>(t, s); break;
+    case 2: launch_tile<2, 2, 1, 2, 2, 4, OUT>(t, s); break;
+    default: launch_tile<1, 2, 1, 2, 2, 6, OUT>(t, s); break;
+    }
+    return true;
+}
+
 // Generic path: one thread per output, any alignment, any even k.
 template <int PK, int OUT>
 __global__ __launch_bounds__(256) void w4a8_generic_kernel(W4A8Args a)
@@ -787,12 +859,11 @@ __global__ __launch_bounds__(256) void w4a8_generic_kernel(W4A8Args a)
         acc += static_cast<uint32_t>(a0 * lo);
         acc += static_cast<uint32_t>(a1 * hi);
     }
-    const float c = a.C ? load_out<OUT>(a.C, static_cast<long long>(gm) * a.ldc + gn) : 0.f;
-    const float b = a.bias ? load_out<OUT>(a.bias, gn) : 0.f;
+    const float c = a.C ? load_out<OUT>(a.C, static_cast<long long>(gm) * a.ldc + gn) : -0.f;
+    const float b = a.bias ? load_out<OUT>(a.bias, gn) : -0.f;
     store_out<OUT>(a.D, static_cast<long long>(gm) * a.ldd + gn,
-                   epilogue_f32(static_cast<int32_t>(acc), static_cast<int32_t>(rsum), a.zp_a[gm],
-                                a.scale_a[gm], a.scale_b[gn], a.C ? &c : nullptr,
-                                a.bias ? &b : nullptr, a.cmin, a.cmax));
+                   w4a8_value(static_cast<int32_t>(acc), static_cast<int32_t>(rsum), a.zp_a[gm],
+                              a.scale_a[gm], a.scale_b[gn], c, b, a.cmin, a.cmax));
 }
 
 template <int kActLoads, int OUT>
@@ -864,6 +935,8 @@ void w4a8_run(size_t m, size_t n, size_t k, const void *A, size_t lda, size_t k_
                       ldd < (1u << 24);
     if (fast && !packed && launch_w4a8_strip<OUT>(a, s)) {
         // decode strip kernel (m = 1, k = 2048 or 4096)
+    } else if (!packed && launch_w4a8_tile<OUT>(a, fast, s)) {
+        // large-tile kernel
     } else if (fast) {
         const unsigned gx = static_cast<unsigned>((n + kNTile - 1) / kNTile);
         const unsigned long long gy = (m + kRowsPerChunk - 1) / kRowsPerChunk;

@@ -1488,18 +1488,6 @@ struct HaloPlan
     int per_xcd;  // tiles per XCD (grid = 8 per_xcd)
 };
 
-// Raw buffer resource (stride 0, 32-bit dwords format): offsets at or past num_records read zeros.
-__device__ __forceinline__ i32x4 raw_rsrc(const void *base, int num_records)
-{
-    const uint64_t b = reinterpret_cast<uint64_t>(base);
-    i32x4 r;
-    r[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(b & 0xffffffffu));
-    r[1] = __builtin_amdgcn_readfirstlane(static_cast<int>((b >> 32) & 0xffffu));
-    r[2] = __builtin_amdgcn_readfirstlane(num_records);
-    r[3] = 0x00020000;
-    return r;
-}
-
 template <int PK>
 __global__ __launch_bounds__(kStreamThreads) void conv_halo_kernel(Int8Args a, HaloPlan hp)
 {

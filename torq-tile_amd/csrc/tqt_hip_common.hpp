@@ -105,6 +105,18 @@ __device__ __forceinline__ void dma_lds16_buf(i32x4 rsrc, int voffset, int8_t *l
 }
 #pragma clang diagnostic pop
 
+// Raw buffer resource (stride 0, 32-bit dwords format): offsets at or past num_records read zeros.
+__device__ __forceinline__ i32x4 raw_rsrc(const void *base, int num_records)
+{
+    const uint64_t b = reinterpret_cast<uint64_t>(base);
+    i32x4 r;
+    r[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(b & 0xffffffffu));
+    r[1] = __builtin_amdgcn_readfirstlane(static_cast<int>((b >> 32) & 0xffffu));
+    r[2] = __builtin_amdgcn_readfirstlane(num_records);
+    r[3] = 0x00020000;
+    return r;
+}
+
 inline bool aligned16(const void *p)
 {
     return (reinterpret_cast<uintptr_t>(p) & 15u) == 0;
@@ -465,6 +477,28 @@ __device__ __forceinline__ void store_out(void *p, long long i, float v)
     }
 }
 
+// Four consecutive elements as one store (i 4-element aligned at p).
+template <int OUT>
+__device__ __forceinline__ void store_out4(void *p, long long i, f32x4 v)
+{
+    if constexpr (OUT == OUT_F32) {
+        *reinterpret_cast<f32x4 *>(static_cast<float *>(p) + i) = v;
+    } else {
+        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+        u16x4 b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (OUT == OUT_F16) {
+                const _Float16 h = static_cast<_Float16>(v[e]);
+                b[e] = v[e] != v[e] ? static_cast<uint16_t>(0x7e00) : __builtin_bit_cast(uint16_t, h);
+            } else {
+                b[e] = f32_to_bf16_bits(v[e]);
+            }
+        }
+        *reinterpret_cast<u16x4 *>(static_cast<uint16_t *>(p) + i) = b;
+    }
+}
+
 // The same conversions through a raw buffer resource: element at byte offset voff + soff (soff
 // wave-uniform); an offset at or past the resource's num_records reads 0 / writes nothing.
 template <int OUT>
@@ -503,6 +537,26 @@ __device__ __forceinline__ void store_out_buf(__amdgpu_buffer_rsrc_t r, uint32_t
         __builtin_amdgcn_raw_buffer_store_b16(bits, r, static_cast<int>(voff),
                                               static_cast<int>(soff), 0);
     }
+}
+
+// reference tqt_kernel_gemm_i8_i4_4x1vl_rvv.h:234-419: zp correction (int32), RNE convert, two
+// separate multiplies, C then bias (separate adds), vfmax then vfmin.
+// C and bias are added always: an absent one is passed as -0, which leaves every value as it is.
+__device__ __forceinline__ float w4a8_value(int32_t acc, int32_t rsum, int32_t zp, float sa,
+                                            float sb, float c, float bias, float cmin, float cmax)
+{
+    // Rounds after every operation: the library is built with -ffp-contract=off, since hipcc
+    // would otherwise fuse a * b + c (__fmul_rn / __fadd_rn do not prevent it).
+    const int32_t v = static_cast<int32_t>(static_cast<uint32_t>(acc) -
+                                           static_cast<uint32_t>(zp) * static_cast<uint32_t>(rsum));
+    float f = __int2float_rn(v);
+    f = __fmul_rn(f, sa);
+    f = __fmul_rn(f, sb);
+    f = __fadd_rn(f, c);
+    f = __fadd_rn(f, bias);
+    f = fmaxf(f, cmin);
+    f = fminf(f, cmax);
+    return f;
 }
 
 // RISC-V vfmax / vfmin on f32 (IEEE 754-2019 maximumNumber / minimumNumber): a NaN operand
