@@ -1,0 +1,123 @@
+"""W4A16 large-tile kernel (many rows, scale blocks that are any multiple of 32, k beyond the
+register kernel): against the CPU oracle and exact f64 math at the edges of its tiles (128 x 256,
+128 x 128, 64 x 128, 32 x 64), at stage remainders, with every block width class (32, 64, 96, 128,
+one block over the whole of k), odd scale strides (a scale is then the upper half of its dword in
+every other row), C, clamps, strides, infinities, and f16 and f32 results."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import tqt_testlib as T
+from test_gpu_parity import check_w4a16
+
+pytestmark = pytest.mark.gpu
+
+
+def _gr():
+    import gpu_run
+
+    return gpu_run
+
+
+def _run_f32(d, lo=-np.inf, hi=np.inf, pad_d=0, pad_s=0):
+    import torch
+
+    g = _gr()
+    A16, Bp, S16, bl = d["A16"], d["Bp"], d["S16"], d["bl"]
+    (m, k), n, nb = A16.shape, Bp.shape[0], S16.shape[1]
+    S = np.full((n, nb + pad_s), 0x7E00, np.uint16)  # NaN beyond the blocks
+    S[:, :nb] = S16
+    dA, dB, dS = g.dev(A16.view(np.int16)), g.dev(Bp), g.dev(S.view(np.int16))
+    C = None if d["C16"] is None else T.bits_f16(d["C16"]).astype(np.float32)
+    bias = None if d["bias16"] is None else T.bits_f16(d["bias16"]).astype(np.float32)
+    dC, dbias = g.dev(C), g.dev(bias)
+    dD = torch.full((m + 1, n + pad_d), 12345.0, dtype=torch.float32, device="cuda:0")
+    g.lib().fn("w4a16f", "run")(m, n, k, bl, g.dp(dA), k, 0, g.dp(dB), k, 0, g.dp(dS), nb + pad_s,
+                                g.dp(dC), n, g.dp(dD), n + pad_d, g.dp(dbias), lo, hi)
+    got = dD.cpu().numpy()
+    assert (got[m:] == 12345.0).all() and (got[:m, n:] == 12345.0).all()
+    return np.ascontiguousarray(got[:m, :n])
+
+
+def _exact(d):
+    """f64 sums and the sum of the terms' magnitudes, C and bias included."""
+    a = T.bits_f16(d["A16"]).astype(np.float64)
+    bl = d["bl"]
+    q = np.empty((d["Bp"].shape[0], a.shape[1]), np.float64)
+    q[:, 0::2] = (d["Bp"] & 15).astype(np.float64) - 8
+    q[:, 1::2] = (d["Bp"] >> 4).astype(np.float64) - 8
+    w = q * np.repeat(T.bits_f16(d["S16"]).astype(np.float64), bl, axis=1)
+    v, mag = a @ w.T, np.abs(a) @ np.abs(w).T
+    for x in (d["C16"], d["bias16"]):
+        if x is not None:
+            f = T.bits_f16(x).astype(np.float64)
+            v, mag = v + f, mag + np.abs(f)
+    return v, mag
+
+
+def _check_f32(got, d, lo=-np.inf, hi=np.inf):
+    """Each block's products and sum round at most bl times (exact products), its scaled value and
+    the accumulation once each, and C, bias and the k groups a few times more: (bl + k / bl + 16)
+    roundings of 2^-24 of the terms' magnitude."""
+    v, mag = _exact(d)
+    k = d["A16"].shape[1]
+    bound = (d["bl"] + k / d["bl"] + 16) * 2.0 ** -24 * mag
+    v = np.clip(v, lo, hi)
+    bad = np.abs(got.astype(np.float64) - v) > bound
+    assert not bad.any(), "%d of %d outputs out of bounds" % (bad.sum(), bad.size)
+
+
+# (m, n, k, bl)
+SHAPES = [
+    (1, 65, 160, 32),        # a single row
+    (300, 400, 32, 32),      # one block of k
+    (520, 130, 96, 96),
+    (31, 130, 864, 32),      # k % 128 == 96
+    (33, 65, 160, 32),
+    (65, 129, 2880, 96),     # blocks that straddle stages
+    (129, 257, 1152, 128),   # odd scale stride (9)
+    (100, 1000, 4416, 64),   # k beyond the register kernel, odd scale stride (69)
+    (300, 1001, 1056, 1056),  # one block over all of k, odd channels
+    (700, 2100, 544, 32),    # 64 x 128 or 128 x 128 tiles
+    (1030, 4100, 320, 64),
+    (2100, 2100, 256, 128),
+    (64, 512, 8192, 32),
+]
+
+
+@pytest.mark.parametrize("m,n,k,bl", SHAPES)
+def test_w4a16_tile_f32(gpu, m, n, k, bl):
+    d = T.gen_w4a16(m, n, k, bl=bl, seed=m + n + k, with_c=bool(m & 1), with_bias=bool(n & 1))
+    lo, hi = (-np.inf, np.inf) if m % 2 else (-3.0, 4.0)
+    _check_f32(_run_f32(d, lo, hi, pad_d=n % 3, pad_s=(m % 2)), d, lo, hi)
+
+
+@pytest.mark.parametrize("m,n,k,bl", SHAPES)
+def test_w4a16_tile_f16(gpu, shim, m, n, k, bl):
+    d = T.gen_w4a16(m, n, k, bl=bl, seed=m * 3 + n + k, with_c=bool(m & 1), with_bias=bool(n & 1))
+    lo, hi = (-65504.0, 65504.0) if m % 2 else (-2.0, 2.5)
+    cmin, cmax = int(T.f16_bits(lo)), int(T.f16_bits(hi))
+    got = _gr().run_w4a16(shim, d, cmin, cmax)
+    exp = T.oracle_w4a16(d["A16"], d["Bp"], d["S16"], bl, d["C16"], d["bias16"], cmin, cmax)
+    check_w4a16(got, exp, d, (lo, hi))
+
+
+@pytest.mark.parametrize("bl", [32, 64])
+def test_w4a16_tile_infinity(gpu, bl):
+    """An infinite activation gives infinite results of its sign, NaN where its weight is 0 (as the
+    oracle's order of operations does), also through the compensated accumulators, and leaves the
+    other rows alone."""
+    m, n, k = 40, 196, 1024 + bl
+    d = T.gen_w4a16(m, n, k, bl=bl, seed=9)
+    d["A16"][7, 100] = 0x7C00
+    d["A16"][9, 1000] = 0xFC00
+    got = _run_f32(d)
+    for row, byte, sign in ((7, 50, 1), (9, 500, -1)):
+        q = (d["Bp"][:, byte] & 15).astype(np.int32) - 8
+        assert np.isnan(got[row, q == 0]).all()
+        assert (got[row, q > 0] == sign * np.inf).all() and (got[row, q < 0] == -sign * np.inf).all()
+    rest = np.ones(m, bool)
+    rest[[7, 9]] = False
+    assert np.isfinite(got[rest]).all()

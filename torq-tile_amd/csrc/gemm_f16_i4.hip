@@ -1,5 +1,8 @@
 // gemm_1xnbias_clamp_f16_f16_qsi4c2t (W4A16, block-quantized int4 weights) on gfx950.
 //
+// Many rows, scale blocks other than 32 wide, or k beyond what the kernels below take (plain
+// layouts): the large-tile kernel of f16_tile.hpp.
+//
 // Two MFMA kernels share the math below: w4a16_chunk_kernel (k % 512 == 0: 16 waves per CU walk
 // k in 512-wide chunks streamed through a shared LDS ring; see its own comment) and
 // w4a16_mfma_kernel (any other k % 128 == 0, k <= 4096). In w4a16_mfma_kernel a workgroup of
@@ -22,6 +25,7 @@
 // oracle's exact operation order (reference test/common/reference_gemm.cpp:132-179).
 #include <type_traits>
 
+#include "f16_tile.hpp"
 #include "tqt_hip_common.hpp"
 #include "tqt_gemm_1xnbias_clamp_f16_f16_qsi4c2t_mfma_gfx950.h"
 #include "tqt_gemm_1xnbias_clamp_f16_f16p_qsi4c2p_mfma_gfx950.h"
@@ -626,6 +630,157 @@ int device_cu_count()
     return cus > 0 ? cus : 1;
 }
 
+// ---------------------------------------------------------------------------------------------
+// Large-tile kernel (f16_tile.hpp): which tile a shape takes, by the same rule as the int8 tiles.
+// A launch is rounds of 256 tiles, one per CU, of fixed + rate * ceil(k / 128) microseconds; the
+// 4-wave tiles also run two to a CU (a pair of rounds at a cost of its own). Measured on MI355X at
+// k 4096 (32 stages), per round of 256 tiles; pair in parentheses:
+//                     32-wide blocks   64-wide       compensated (f32 results, 32-wide blocks)
+//   128 x 256         110              80
+//   128 x 128         58               50
+//   64 x 128          35 (64)          33 (51)       49 (88)
+//   32 x 64           18 (25)          16 (24)       22 (31)
+// Against the kernels above at 4096 x 4096, 32-wide blocks, f16 results: 12.6 us for 32 rows there
+// (18.7 here), 23.2 for 64 (18.7), 44.3 for 128 (18.8).
+// ---------------------------------------------------------------------------------------------
+struct F16TileShape
+{
+    int bm, bn;
+    float fixed, stage;            // us of one round
+    float pair_fixed, pair_stage;  // us of two
+};
+constexpr int kF16Shapes = 4;
+constexpr F16TileShape kF16Tiles[3][kF16Shapes] = {
+    // 32-wide blocks
+    {{128, 256, 9.f, 3.1f, 18.f, 6.2f}, {128, 128, 6.f, 1.6f, 12.f, 3.2f},
+     {64, 128, 4.5f, .95f, 5.f, 1.85f}, {32, 64, 4.2f, .44f, 5.f, .61f}},
+    // blocks of a multiple of 64
+    {{128, 256, 9.f, 2.2f, 18.f, 4.4f}, {128, 128, 6.f, 1.4f, 12.f, 2.8f},
+     {64, 128, 4.5f, .9f, 5.f, 1.45f}, {32, 64, 4.2f, .38f, 5.f, .58f}},
+    // compensated: the registers of the two larger tiles do not suffice
+    {{0, 0, 0.f, 0.f, 0.f, 0.f}, {0, 0, 0.f, 0.f, 0.f, 0.f},
+     {64, 128, 4.5f, 1.4f, 5.f, 2.6f}, {32, 64, 4.2f, .57f, 5.f, .8f}}};
+
+template <int MI, int WGN, int KS, int NS, int SPB, int COMP, int OUT>
+void launch_f16_tile(F16TileArgs t, hipStream_t s)
+{
+    constexpr int BM = 32 * MI, BN = 32 * WGN;
+    t.tiles_m = (t.M + BM - 1) / BM;
+    t.tiles_n = (t.N + BN - 1) / BN;
+    const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;
+    TQT_REQUIRE(tiles < (1ll << 28), "grid too large");
+    t.per_xcd = static_cast<int>((tiles + 7) / 8);
+    hipLaunchKernelGGL((w4a16_tile_kernel<MI, WGN, KS, NS, SPB, COMP, OUT>),
+                       dim3(8 * static_cast<unsigned>(t.per_xcd)), dim3(64 * WGN * KS), 0, s, t);
+}
+
+template <int SPB, int OUT>
+void launch_f16_tile_shape(int shape, const F16TileArgs &t, hipStream_t s)
+{
+    switch (shape) {
+    case 0: launch_f16_tile<4, 8, 1, 3, SPB, 0, OUT>(t, s); break;
+    case 1: launch_f16_tile<4, 4, 2, 3, SPB, 0, OUT>(t, s); break;
+    case 2: launch_f16_tile<2, 4, 1, 3, SPB, 0, OUT>(t, s); break;
+    default: launch_f16_tile<1, 2, 2, 6, SPB, 0, OUT>(t, s); break;
+    }
+}
+
+// f32 results with 32-wide blocks. One compensation per block up to k 1536 and per two blocks past
+// it: relative error against 64 bits 4.5e-8 and 4.9e-8 at every k, where the kernels above have
+// 4.4e-8 at k 512, 4.8e-8 at 1024, 5.4e-8 at 2048 and 6.5e-8 at 4096, and plain accumulators
+// 6.2e-8 to 2.7e-7 (64 x 128 tiles at k 4096: 64 us a pair of rounds plain, 88 and 112 compensated).
+inline void launch_f16_tile_comp(int shape, const F16TileArgs &t, hipStream_t s)
+{
+    const bool every = t.K < 1536;
+    if (shape == 2) {
+        if (every) {
+            launch_f16_tile<2, 4, 1, 3, 1, 1, OUT_F32>(t, s);
+        } else {
+            launch_f16_tile<2, 4, 1, 3, 1, 2, OUT_F32>(t, s);
+        }
+    } else {
+        if (every) {
+            launch_f16_tile<1, 2, 2, 6, 1, 1, OUT_F32>(t, s);
+        } else {
+            launch_f16_tile<1, 2, 2, 6, 1, 2, OUT_F32>(t, s);
+        }
+    }
+}
+
+// The tile kernel for plain layouts with 16-byte aligned rows and scale blocks of whole 32-k
+// groups; false when it does not apply (its offsets are 32 bits from a tile's first row) or
+// another kernel's estimate (other_us, 0: no other kernel but the generic one) is lower.
+template <int OUT>
+bool launch_w4a16_tile(const W4A16Args &a, float other_us, hipStream_t s)
+{
+    constexpr long long kElem = OUT == OUT_F32 ? 4 : 2;
+    // Under a stage of k and few outputs the generic kernel takes a few microseconds and sums in
+    // the oracle's order.
+    if (a.K < 128 && static_cast<long long>(a.M) * a.N <= 65536) {
+        return false;
+    }
+    // One chunk of k with f32 results: the chunk-stream kernel's sixteen f64-summed blocks are the
+    // more exact (4.5e-8 against 4.7e-8).
+    if (OUT == OUT_F32 && a.K == kCsK && other_us > 0.f) {
+        return false;
+    }
+    if (a.K == 0 || a.bl % 32 != 0 || a.lda % 8 != 0 || a.bstride % 16 != 0 || !aligned16(a.A) ||
+        !aligned16(a.B) || a.lda >= (1 << 22) || a.bstride >= (1 << 22) || a.ldsb >= (1 << 22) ||
+        a.ldd * kElem >= (1 << 23) || (a.C && a.ldc * kElem >= (1 << 23))) {
+        return false;
+    }
+    const int variant = a.bl % 64 == 0 ? 1 : (OUT == OUT_F32 ? 2 : 0);
+    const float stages = static_cast<float>((a.K + 127) / 128);
+    int best = -1;
+    float best_us = 0.f;
+    for (int i = variant == 2 ? 2 : 0; i < kF16Shapes; ++i) {
+        const F16TileShape &p = kF16Tiles[variant][i];
+        const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
+                                ((a.N + p.bn - 1) / p.bn);
+        const long long rounds = (tiles + kTileCUs - 1) / kTileCUs;
+        const float us =
+            static_cast<float>(rounds / 2) * (p.pair_fixed + p.pair_stage * stages) +
+            static_cast<float>(rounds % 2) * (p.fixed + p.stage * stages);
+        if (best < 0 || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    if (other_us > 0.f && other_us <= best_us) {
+        return false;
+    }
+    F16TileArgs t = {};
+    t.M = a.M;
+    t.N = a.N;
+    t.K = a.K;
+    t.A = a.A;
+    t.lda = a.lda;
+    t.B = a.B;
+    t.bstride = a.bstride;
+    t.scale_b = a.scale_b;
+    t.ldsb = a.ldsb;
+    t.C = a.C;
+    t.ldc = a.ldc;
+    t.D = a.D;
+    t.ldd = a.ldd;
+    t.bias = a.bias;
+    t.cmin = a.cmin;
+    t.cmax = a.cmax;
+    t.bl = a.bl;
+    t.nblocks = a.K / a.bl;
+    // the clamp's answer to a NaN is that of the kernel that takes the shape otherwise: the lower
+    // bound from the 32-wide-block kernels (fmax), NaN from the generic one (compare and select)
+    t.nan_to_min = other_us > 0.f;
+    if (variant == 1) {
+        launch_f16_tile_shape<2, OUT>(best, t, s);
+    } else if constexpr (OUT == OUT_F32) {
+        launch_f16_tile_comp(best, t, s);
+    } else {
+        launch_f16_tile_shape<1, OUT>(best, t, s);
+    }
+    return true;
+}
+
 // Shared body of the W4A16 runs. OUT: OUT_F16 (C, bias, D f16) or OUT_F32 (C, bias, D f32);
 // the clamp bounds arrive widened to f32. `packed`: A (f16 rows) and B (int4 rows,
 // fragment-ordered) are in the packed layout; k_idx_a / k_idx_b apply the packers' tail rule.
@@ -682,7 +837,24 @@ void w4a16_run(size_t m, size_t n, size_t k, size_t bl, const void *A, size_t ld
     // bl 32 and k % 512 == 0: the chunk-stream kernel
     const bool chunk = bl == 32 && k % kCsK == 0 && k >= kCsK && layout_fast && ldsb % 8 == 0 &&
                        aligned16(A) && aligned16(B) && aligned16(scale_b);
+    // Microseconds of the chunk-stream and register kernels, from measurements at one and four
+    // tiles per workgroup: every 32 rows are a pass of their own over the weights.
+    const long long row_groups = static_cast<long long>((m + kMRows - 1) / kMRows);
+    float other_us = 0.f;
     if (chunk) {
+        const long long wgs = a.ntiles <= kTileCUs ? a.ntiles : (a.ntiles + kCsTiles - 1) / kCsTiles;
+        const long long nwg = a.ntiles > kTileCUs && wgs < kTileCUs ? kTileCUs : wgs;
+        other_us = static_cast<float>((row_groups * nwg + kTileCUs - 1) / kTileCUs) *
+                   (3.5f + 0.97f * static_cast<float>(a.K / kCsK));
+    } else if (fast) {
+        const long long gx = a.ntiles < kTileCUs ? a.ntiles : kTileCUs;
+        const float strip = static_cast<float>(a.ntiles) / static_cast<float>(gx) - 1.f;
+        other_us = static_cast<float>((row_groups * gx + kTileCUs - 1) / kTileCUs) *
+                   (3.5f + static_cast<float>(a.K) * (0.002f + 0.0006f * strip));
+    }
+    if (!packed && launch_w4a16_tile<OUT>(a, other_us, s)) {
+        // large-tile kernel
+    } else if (chunk) {
         const int cus = device_cu_count();  // the current device, per call (no cached state)
         const long long need = (a.ntiles + kCsTiles - 1) / kCsTiles;
         const long long nwg = need > cus ? need : (a.ntiles < cus ? a.ntiles : cus);

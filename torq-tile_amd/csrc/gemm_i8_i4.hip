@@ -751,8 +751,6 @@ bool launch_w4a8_qstrip(const W4A8Args &a, const float *X, int8_t *Aq, float *sa
 // 32, 23.0 at 48, against 12.2-12.8 for the tiles; 4096 x 4096: 9.7 at 48 and 27.1 at 200, against
 // 12.5 and 12.8).
 // ---------------------------------------------------------------------------------------------
-constexpr int kTileCUs = 256;  // compute units of an MI355X
-
 struct TileShape
 {
     int bm, bn;

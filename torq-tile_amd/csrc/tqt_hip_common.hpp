@@ -103,6 +103,40 @@ __device__ __forceinline__ void dma_lds16_buf(i32x4 rsrc, int voffset, int8_t *l
     (void)lds;
 #endif
 }
+
+// The same with a wave-uniform byte offset soffset added (not part of the range check: for loads
+// known to be in range).
+__device__ __forceinline__ void dma_lds16_buf_s(i32x4 rsrc, int voffset, int soffset, int8_t *lds)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t base =
+        __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %3 offen lds" ::"v"(voffset),
+                 "s"(rsrc), "s"(base), "s"(soffset)
+                 : "memory", "m0");
+#else
+    (void)rsrc;
+    (void)voffset;
+    (void)soffset;
+    (void)lds;
+#endif
+}
+
+// The same with 4 bytes per lane (lane i's dword at lds + 4 i).
+__device__ __forceinline__ void dma_lds4_buf(i32x4 rsrc, int voffset, int8_t *lds)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t base =
+        __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds)));
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(voffset),
+                 "s"(rsrc), "s"(base)
+                 : "memory", "m0");
+#else
+    (void)rsrc;
+    (void)voffset;
+    (void)lds;
+#endif
+}
 #pragma clang diagnostic pop
 
 // Raw buffer resource (stride 0, 32-bit dwords format): offsets at or past num_records read zeros.
