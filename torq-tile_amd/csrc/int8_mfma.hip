@@ -9,7 +9,9 @@
 //   igemmcf_mx1bias_reqi32toi8_clamp_qai8_qsi8dx_qai8   (B gathered from an NCDHW image)
 // and their packed siblings.
 //
-// Four kernels, chosen per call:
+// Five kernels, chosen per call:
+//   * int8_skinny_kernel (int8_skinny.hpp; B = [n, k], W8A8 static and dynamic, few rows: decode):
+//     16 channels per workgroup, k split over its waves, each with a ring of its own;
 //   * conv_halo_kernel (igemmcl, plain or packed weights, 3 x 3 "same" convolution with stride 1
 //     and 128 channels per group: the benchmark's): each workgroup loads the input rows its 256
 //     output pixels touch into LDS once and forms the nine taps from them (described at the
@@ -23,7 +25,7 @@
 //     LDS tiles, v_mfma_i32_16x16x64_i8;
 //   * int8_generic_kernel: one thread per output for unaligned pointers or strides, k not a
 //     multiple of 16, or channel counts not a multiple of 16.
-// All four accumulate exactly in int32 and fuse the epilogue (C, bias, requantization,
+// All accumulate exactly in int32 and fuse the epilogue (C, bias, requantization,
 // saturation, clamp) into the store.
 #include <type_traits>
 
@@ -1972,11 +1974,25 @@ bool launch_small_clamp(const Int8Args &a, hipStream_t stream)
     return true;
 }
 
+}  // namespace
+}  // namespace tqt
+
+#include "int8_skinny.hpp"
+
+namespace tqt {
+namespace {
+
 template <int AM, int BMd, int EPI, int PK = PK_NONE>
 void launch_int8(const Int8Args &a, bool fast, hipStream_t stream, const char *where)
 {
     if (a.M <= 0 || a.N <= 0) {
         return;
+    }
+    if constexpr (BMd == B_NK && AM == A_MATRIX && (is_dyn(EPI) || EPI == EPI_REQUANT_I8)) {
+        if (fast && launch_skinny<EPI, PK>(a, stream)) {
+            check_launch(where);
+            return;
+        }
     }
     // The streaming kernel takes plain (or packed) matrices and the implicit convolution whose
     // group channel count is a multiple of its 128-byte stage (conv_bytes > 0, set by the
