@@ -9,7 +9,9 @@
 //   igemmcf_mx1bias_reqi32toi8_clamp_qai8_qsi8dx_qai8   (B gathered from an NCDHW image)
 // and their packed siblings.
 //
-// Five kernels, chosen per call:
+// Six kernels, chosen per call:
+//   * w8a8_tile_kernel (w8a8_tile.hpp; B = [n, k], W8A8 static and dynamic, large outputs): tiles of
+//     256 x 256 and 128 x 128;
 //   * int8_skinny_kernel (int8_skinny.hpp; B = [n, k], W8A8 static and dynamic, few rows: decode):
 //     16 channels per workgroup, k split over its waves, each with a ring of its own;
 //   * conv_halo_kernel (igemmcl, plain or packed weights, 3 x 3 "same" convolution with stride 1
@@ -29,6 +31,7 @@
 // saturation, clamp) into the store.
 #include <type_traits>
 
+#include "int8_tile.hpp"
 #include "tqt_hip_common.hpp"
 #include "tqt_gemm_1xnbias_reqi32toi8_clamp_qai8_qai8_qsi8cxt_mfma_gfx950.h"
 #include "tqt_gemm_clamp_i32_i8_i8_mfma_gfx950.h"
@@ -160,16 +163,15 @@ __device__ uint32_t dyn_exact_acc(const Int8Args &a, int gm, int gn, int32_t zp)
 // rounded to f16, + the f16 bias in f16, then the bounds. Every step rounds once (the library is
 // built without contraction).
 template <int EPI>
-__device__ __forceinline__ void dyn_finish_v(const Int8Args &a, int gn, long long drow, uint32_t x,
-                                             float sb, float sa, float fb)
+__device__ __forceinline__ float dyn_value(const Int8Args &a, uint32_t x, float sb, float sa,
+                                           float fb)
 {
     const float sigma = __fmul_rn(sb, sa);
     const float f = __fmul_rn(static_cast<float>(static_cast<int32_t>(x)), sigma);
     if constexpr (EPI == EPI_DYN_F32) {
         float v = __fadd_rn(f, fb);
         v = rv_fmaxf(v, a.fcmin);
-        v = rv_fminf(v, a.fcmax);
-        static_cast<float *>(a.D)[drow * a.ldd + gn] = v;
+        return rv_fminf(v, a.fcmax);
     } else {
         // The product must be rounded to f32 before the f16 conversion (vfmul then vfncvt):
         // without this register barrier the compiler folds both into one v_fma_mixlo_f16, which
@@ -180,9 +182,16 @@ __device__ __forceinline__ void dyn_finish_v(const Int8Args &a, int gn, long lon
         const _Float16 b = static_cast<_Float16>(fb);  // exact: fb holds a binary16 value
         const _Float16 hs = h + b;  // one binary16 rounding
         float v = rv_fmaxf(static_cast<float>(hs), a.fcmin);  // exact on binary16 values
-        v = rv_fminf(v, a.fcmax);
-        store_out<OUT_F16>(a.D, drow * a.ldd + gn, v);
+        return rv_fminf(v, a.fcmax);
     }
+}
+
+template <int EPI>
+__device__ __forceinline__ void dyn_finish_v(const Int8Args &a, int gn, long long drow, uint32_t x,
+                                             float sb, float sa, float fb)
+{
+    store_out<EPI == EPI_DYN_F32 ? OUT_F32 : OUT_F16>(a.D, drow * a.ldd + gn,
+                                                      dyn_value<EPI>(a, x, sb, sa, fb));
 }
 
 __device__ __forceinline__ bool dyn_zp_in_range(int32_t zp)
@@ -1978,6 +1987,7 @@ bool launch_small_clamp(const Int8Args &a, hipStream_t stream)
 }  // namespace tqt
 
 #include "int8_skinny.hpp"
+#include "w8a8_tile.hpp"
 
 namespace tqt {
 namespace {
@@ -1989,7 +1999,7 @@ void launch_int8(const Int8Args &a, bool fast, hipStream_t stream, const char *w
         return;
     }
     if constexpr (BMd == B_NK && AM == A_MATRIX && (is_dyn(EPI) || EPI == EPI_REQUANT_I8)) {
-        if (fast && launch_skinny<EPI, PK>(a, stream)) {
+        if (fast && (launch_skinny<EPI, PK>(a, stream) || launch_w8a8_tile<EPI, PK>(a, stream))) {
             check_launch(where);
             return;
         }
