@@ -446,12 +446,18 @@ bool launch_w8a8_tile(const Int8Args &a, hipStream_t stream)
     };
     const long long r128 = rounds(128), r256 = rounds(256);
     const float fr = static_cast<float>(r128);
-    const float stream_us = fr * (kDyn ? 3.f + 1.0f * n : 3.f + 0.67f * n);
+    // k not a multiple of 128 has the double-buffered kernel instead of the stream kernel, which one
+    // nearly full round of large tiles beats too (1000 x 4096 x 4112: 32.5 us, 41 there) and a half
+    // full one does not (512 x 4096 x 4112: 30 us, 27 there)
+    const bool other = a.K % kTileK != 0;
+    const float stream_us =
+        fr * (other ? 3.f + 1.2f * n : (kDyn ? 3.f + 1.0f * n : 3.f + 0.67f * n));
     const float mid_us =
         static_cast<float>(r128 / 2) * (kDyn ? 6.f + 1.5f * n : 5.f + 1.2f * n) +
         static_cast<float>(r128 % 2) * (kDyn ? 6.f + 0.9f * n : 4.f + 0.7f * n);
     const float big_us = static_cast<float>(r256) * (kDyn ? 20.f + 1.8f * n : 14.f + 1.5f * n);
-    if (r128 < 2 || (stream_us <= mid_us && stream_us <= big_us)) {
+    const long long t128 = static_cast<long long>((a.M + 127) / 128) * ((a.N + 127) / 128);
+    if (t128 <= (other ? 3 * kTileCUs / 4 : kTileCUs) || (stream_us <= mid_us && stream_us <= big_us)) {
         return false;
     }
     if (big_us < mid_us) {
