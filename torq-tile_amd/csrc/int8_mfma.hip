@@ -9,7 +9,9 @@
 //   igemmcf_mx1bias_reqi32toi8_clamp_qai8_qsi8dx_qai8   (B gathered from an NCDHW image)
 // and their packed siblings.
 //
-// Six kernels, chosen per call:
+// Seven kernels, chosen per call:
+//   * conv_cf_kernel (conv_cf.hpp; igemmcf with plain weights, 1, 9 or 25 taps, channels a multiple of
+//     16): both operands turned to channel-last in LDS once per workgroup;
 //   * w8a8_tile_kernel (w8a8_tile.hpp; B = [n, k], W8A8 static and dynamic, large outputs): tiles of
 //     256 x 256 and 128 x 128;
 //   * int8_skinny_kernel (int8_skinny.hpp; B = [n, k], W8A8 static and dynamic, few rows: decode):
@@ -1988,6 +1990,7 @@ bool launch_small_clamp(const Int8Args &a, hipStream_t stream)
 
 #include "int8_skinny.hpp"
 #include "w8a8_tile.hpp"
+#include "conv_cf.hpp"
 
 namespace tqt {
 namespace {
@@ -2027,6 +2030,12 @@ void launch_int8(const Int8Args &a, bool fast, hipStream_t stream, const char *w
     if constexpr (BMd == B_NK && AM == A_CONV_CL && EPI == EPI_REQUANT_I8) {
         if (fast && a.conv_bytes > 0 && a.cv.ICg % kSK == 0 && stream_offsets_fit(a, 1)) {
             launch_stream<EPI, PK, true>(a, stream);
+            check_launch(where);
+            return;
+        }
+    }
+    if constexpr (AM == A_MATRIX && BMd == B_CF && EPI == EPI_REQUANT_ROW && PK == PK_NONE) {
+        if (fast && launch_conv_cf(a, stream)) {
             check_launch(where);
             return;
         }
