@@ -25,6 +25,7 @@
 // oracle's exact operation order (reference test/common/reference_gemm.cpp:132-179).
 #include <type_traits>
 
+#include "f16_skinny.hpp"
 #include "f16_tile.hpp"
 #include "tqt_hip_common.hpp"
 #include "tqt_gemm_1xnbias_clamp_f16_f16_qsi4c2t_mfma_gfx950.h"
@@ -707,48 +708,11 @@ inline void launch_f16_tile_comp(int shape, const F16TileArgs &t, hipStream_t s)
     }
 }
 
-// The tile kernel for plain layouts with 16-byte aligned rows and scale blocks of whole 32-k
-// groups; false when it does not apply (its offsets are 32 bits from a tile's first row) or
-// another kernel's estimate (other_us, 0: no other kernel but the generic one) is lower.
-template <int OUT>
-bool launch_w4a16_tile(const W4A16Args &a, float other_us, hipStream_t s)
+// The tile kernels' arguments. nan_to_min: the clamp's answer to a NaN is that of the kernel that
+// takes the shape otherwise - the lower bound from the 32-wide-block kernels (fmax), NaN from the
+// generic one (compare and select).
+inline F16TileArgs tile_args(const W4A16Args &a, bool nan_to_min)
 {
-    constexpr long long kElem = OUT == OUT_F32 ? 4 : 2;
-    // Under a stage of k and few outputs the generic kernel takes a few microseconds and sums in
-    // the oracle's order.
-    if (a.K < 128 && static_cast<long long>(a.M) * a.N <= 65536) {
-        return false;
-    }
-    // One chunk of k with f32 results: the chunk-stream kernel's sixteen f64-summed blocks are the
-    // more exact (4.5e-8 against 4.7e-8).
-    if (OUT == OUT_F32 && a.K == kCsK && other_us > 0.f) {
-        return false;
-    }
-    if (a.K == 0 || a.bl % 32 != 0 || a.lda % 8 != 0 || a.bstride % 16 != 0 || !aligned16(a.A) ||
-        !aligned16(a.B) || a.lda >= (1 << 22) || a.bstride >= (1 << 22) || a.ldsb >= (1 << 22) ||
-        a.ldd * kElem >= (1 << 23) || (a.C && a.ldc * kElem >= (1 << 23))) {
-        return false;
-    }
-    const int variant = a.bl % 64 == 0 ? 1 : (OUT == OUT_F32 ? 2 : 0);
-    const float stages = static_cast<float>((a.K + 127) / 128);
-    int best = -1;
-    float best_us = 0.f;
-    for (int i = variant == 2 ? 2 : 0; i < kF16Shapes; ++i) {
-        const F16TileShape &p = kF16Tiles[variant][i];
-        const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
-                                ((a.N + p.bn - 1) / p.bn);
-        const long long rounds = (tiles + kTileCUs - 1) / kTileCUs;
-        const float us =
-            static_cast<float>(rounds / 2) * (p.pair_fixed + p.pair_stage * stages) +
-            static_cast<float>(rounds % 2) * (p.fixed + p.stage * stages);
-        if (best < 0 || us < best_us) {
-            best = i;
-            best_us = us;
-        }
-    }
-    if (other_us > 0.f && other_us <= best_us) {
-        return false;
-    }
     F16TileArgs t = {};
     t.M = a.M;
     t.N = a.N;
@@ -768,17 +732,120 @@ bool launch_w4a16_tile(const W4A16Args &a, float other_us, hipStream_t s)
     t.cmax = a.cmax;
     t.bl = a.bl;
     t.nblocks = a.K / a.bl;
-    // the clamp's answer to a NaN is that of the kernel that takes the shape otherwise: the lower
-    // bound from the 32-wide-block kernels (fmax), NaN from the generic one (compare and select)
-    t.nan_to_min = other_us > 0.f;
-    if (variant == 1) {
-        launch_f16_tile_shape<2, OUT>(best, t, s);
-    } else if constexpr (OUT == OUT_F32) {
-        launch_f16_tile_comp(best, t, s);
-    } else {
-        launch_f16_tile_shape<1, OUT>(best, t, s);
+    t.nan_to_min = nan_to_min;
+    return t;
+}
+
+// Layouts the tile kernels take: 16-byte aligned rows, scale blocks of whole 32-k groups, strides
+// within their 32-bit offsets.
+template <int OUT>
+bool tile_layout(const W4A16Args &a)
+{
+    constexpr long long kElem = OUT == OUT_F32 ? 4 : 2;
+    return a.K > 0 && a.bl % 32 == 0 && a.lda % 8 == 0 && a.bstride % 16 == 0 && aligned16(a.A) &&
+           aligned16(a.B) && a.lda < (1 << 22) && a.bstride < (1 << 22) && a.ldsb < (1 << 22) &&
+           a.ldd * kElem < (1 << 23) && (!a.C || a.ldc * kElem < (1 << 23));
+}
+
+// Microseconds of the few-row kernel (f16_skinny.hpp), 0 where it does not apply: a fixed part and
+// the 16-channel strips that one CU streams one after another, more slowly with the activation rows
+// that each strip loads too. At k 4096 and one row: 256 strips 6.5, 512 8.7, 768 10.5, 896 13.5 (four
+// on some CUs); 1792 strips at k 8192 34.5; with 16 rows 7.4, 12.3, -, 17.7 and 48.5.
+template <int OUT>
+float w4a16_skinny_us(const W4A16Args &a)
+{
+    if (a.M > 16 || a.K < 128 || !tile_layout<OUT>(a)) {
+        return 0.f;
     }
-    return true;
+    const int rounds = (a.ntiles + kTileCUs - 1) / kTileCUs;
+    return 4.3f + 2.15f / 4096.f * static_cast<float>(rounds) * static_cast<float>(a.K) *
+                      (1.f + 0.0022f * static_cast<float>(a.M * a.M));
+}
+
+template <int OUT>
+void launch_w4a16_skinny(const W4A16Args &a, bool nan_to_min, hipStream_t s)
+{
+    F16SkinnyArgs f = {};
+    f.t = tile_args(a, nan_to_min);
+    f.bdiv = static_cast<uint32_t>(a.bl / 32);
+    const dim3 grid(static_cast<unsigned>(a.ntiles));
+    // More than two strips a CU: half the waves and one block in flight each, so that four are
+    // resident together (1 x 14336 x 4096: 13.5 us, 14.1 with eight waves; 1 x 4096 x 4096: 7.2 and
+    // 6.6).
+    if (a.ntiles > 2 * kTileCUs) {
+        const dim3 block(256);
+        if (a.M <= 2) {
+            hipLaunchKernelGGL((w4a16_skinny_kernel<4, 1, 1, OUT>), grid, block, 0, s, f);
+        } else if (a.M <= 8) {
+            hipLaunchKernelGGL((w4a16_skinny_kernel<4, 4, 1, OUT>), grid, block, 0, s, f);
+        } else {
+            hipLaunchKernelGGL((w4a16_skinny_kernel<4, 8, 1, OUT>), grid, block, 0, s, f);
+        }
+    } else {
+        const dim3 block(512);
+        if (a.M <= 2) {
+            hipLaunchKernelGGL((w4a16_skinny_kernel<8, 1, 2, OUT>), grid, block, 0, s, f);
+        } else if (a.M <= 8) {
+            hipLaunchKernelGGL((w4a16_skinny_kernel<8, 4, 1, OUT>), grid, block, 0, s, f);
+        } else {
+            hipLaunchKernelGGL((w4a16_skinny_kernel<8, 8, 1, OUT>), grid, block, 0, s, f);
+        }
+    }
+}
+
+// Microseconds of the best tile shape for plain layouts with 16-byte aligned rows and scale blocks
+// of whole 32-k groups, and that shape; 0 where the kernel does not apply (its offsets are 32 bits
+// from a tile's first row). other_us: the chunk-stream or register kernel's, 0 without one.
+struct F16TilePick
+{
+    float us;
+    int variant, shape;
+};
+
+template <int OUT>
+F16TilePick w4a16_tile_pick(const W4A16Args &a, float other_us)
+{
+    F16TilePick best = {0.f, 0, 0};
+    // Under a stage of k and few outputs the generic kernel takes a few microseconds and sums in
+    // the oracle's order.
+    if (a.K < 128 && static_cast<long long>(a.M) * a.N <= 65536) {
+        return best;
+    }
+    // One chunk of k with f32 results: the chunk-stream kernel's sixteen f64-summed blocks are the
+    // more exact (4.5e-8 against 4.7e-8).
+    if ((OUT == OUT_F32 && a.K == kCsK && other_us > 0.f) || !tile_layout<OUT>(a)) {
+        return best;
+    }
+    best.variant = a.bl % 64 == 0 ? 1 : (OUT == OUT_F32 ? 2 : 0);
+    const float stages = static_cast<float>((a.K + 127) / 128);
+    for (int i = best.variant == 2 ? 2 : 0; i < kF16Shapes; ++i) {
+        const F16TileShape &p = kF16Tiles[best.variant][i];
+        const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
+                                ((a.N + p.bn - 1) / p.bn);
+        const long long rounds = (tiles + kTileCUs - 1) / kTileCUs;
+        const float us =
+            static_cast<float>(rounds / 2) * (p.pair_fixed + p.pair_stage * stages) +
+            static_cast<float>(rounds % 2) * (p.fixed + p.stage * stages);
+        if (best.us == 0.f || us < best.us) {
+            best.shape = i;
+            best.us = us;
+        }
+    }
+    return best;
+}
+
+template <int OUT>
+void launch_w4a16_tile(const W4A16Args &a, const F16TilePick &pick, bool nan_to_min,
+                       hipStream_t s)
+{
+    const F16TileArgs t = tile_args(a, nan_to_min);
+    if (pick.variant == 1) {
+        launch_f16_tile_shape<2, OUT>(pick.shape, t, s);
+    } else if constexpr (OUT == OUT_F32) {
+        launch_f16_tile_comp(pick.shape, t, s);
+    } else {
+        launch_f16_tile_shape<1, OUT>(pick.shape, t, s);
+    }
 }
 
 // Shared body of the W4A16 runs. OUT: OUT_F16 (C, bias, D f16) or OUT_F32 (C, bias, D f32);
@@ -852,8 +919,14 @@ void w4a16_run(size_t m, size_t n, size_t k, size_t bl, const void *A, size_t ld
         other_us = static_cast<float>((row_groups * gx + kTileCUs - 1) / kTileCUs) *
                    (3.5f + static_cast<float>(a.K) * (0.002f + 0.0006f * strip));
     }
-    if (!packed && launch_w4a16_tile<OUT>(a, other_us, s)) {
-        // large-tile kernel
+    const F16TilePick tile = packed ? F16TilePick{0.f, 0, 0} : w4a16_tile_pick<OUT>(a, other_us);
+    const float skinny_us = packed ? 0.f : w4a16_skinny_us<OUT>(a);
+    const bool listed = other_us > 0.f;
+    if (skinny_us > 0.f && (!listed || skinny_us < other_us) &&
+        (tile.us == 0.f || skinny_us < tile.us)) {
+        launch_w4a16_skinny<OUT>(a, listed, s);
+    } else if (tile.us > 0.f && (!listed || tile.us < other_us)) {
+        launch_w4a16_tile<OUT>(a, tile, listed, s);
     } else if (chunk) {
         const int cus = device_cu_count();  // the current device, per call (no cached state)
         const long long need = (a.ntiles + kCsTiles - 1) / kCsTiles;
