@@ -32,6 +32,7 @@
 // correction, two scale multiplies, C, bias, clamp; no FMA) runs per output.
 #include <cfloat>
 
+#include "int4_skinny.hpp"
 #include "int8_tile.hpp"
 #include "tqt_hip_common.hpp"
 #include "tqt_gemm_1xnbias_clamp_f32_qai8dx_qsi4cxt_mfma_gfx950.h"
@@ -772,17 +773,8 @@ void launch_tile(TileArgs t, hipStream_t s)
                        dim3(8 * static_cast<unsigned>(t.per_xcd)), dim3(64 * WGM * WGN * KS), 0, s, t);
 }
 
-// The tile kernel for plain layouts whose rows are whole 32-k groups of aligned bytes; false when
-// it does not apply (the kernel's offsets are 32 bits from a tile's first row) or the k-split
-// kernel, if it does (`ksplit`), is the faster one.
-template <int OUT>
-bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
+inline TileArgs tile_args(const W4A8Args &a)
 {
-    if (a.K % 32 != 0 || a.K == 0 || a.K > 65536 || a.lda % 16 != 0 ||
-        a.bstride % 16 != 0 || !aligned16(a.A) || !aligned16(a.B) || a.lda >= (1 << 22) ||
-        a.bstride >= (1 << 22)) {
-        return false;
-    }
     TileArgs t = {};
     t.M = a.M;
     t.N = a.N;
@@ -801,10 +793,21 @@ bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
     t.scale_a = a.scale_a;
     t.zp_a = a.zp_a;
     t.scale_b = a.scale_b;
-    constexpr int kElem = OUT == OUT_F32 ? 4 : 2;
-    t.vec_d = a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.D) % (4 * kElem) == 0;
+    return t;
+}
+
+// Layouts the tile and few-row kernels take: whole 32-k groups, 16-byte aligned rows, strides within
+// their 32-bit offsets, sums of 16 (q - 8) a within an int32.
+inline bool tile_layout(const W4A8Args &a)
+{
+    return a.K % 32 == 0 && a.K > 0 && a.K <= 65536 && a.lda % 16 == 0 && a.bstride % 16 == 0 &&
+           aligned16(a.A) && aligned16(a.B) && a.lda < (1 << 22) && a.bstride < (1 << 22);
+}
+
+// Microseconds of the cheapest tile shape, and which it is.
+inline float w4a8_tile_us(const W4A8Args &a, int &best)
+{
     const float stages = static_cast<float>((a.K + kTileK - 1) / kTileK);
-    int best = 0;
     float best_us = 0.f;
     for (int i = 0; i < 4; ++i) {
         const TileShape &p = kTileShapes[i];
@@ -817,6 +820,70 @@ bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
             best_us = us;
         }
     }
+    return best_us;
+}
+
+// Few rows (int4_skinny.hpp); false where it does not apply or is the slower one. Measured on
+// MI355X (us, weights partly cached; the k-split or tile kernel in parentheses): up to 8 rows it
+// wins at every size - 8 x 4096 x 11008 7.4 (8.1), 4 x 896 x 13792 5.9 (30.8), 8 x 28672 x 8192 22.5
+// (23.1). With more rows the activations weigh as much as the weights and each 16-channel strip
+// reloads them: 9 x 5120 x 12544 10.7 (15.1), 16 x 11008 x 4096 6.9 (12.3), 16 x 28672 x 8192 26.7
+// (24), 32 x 4096 x 4096 5.8 (8.0), 32 x 11008 x 4096 11.1 (12.7), 32 x 28672 x 8192 35 (24).
+// Four waves a workgroup where a CU gets more than two strips (16 x 11008 x 4096 6.9, 8.4 with
+// eight) or k leaves eight little to do (1 x 5504 x 1024 3.2, 4.0); eight stream one strip faster
+// (4 x 896 x 13792 5.9, 8.4 with four).
+template <int OUT>
+bool launch_w4a8_skinny(const W4A8Args &a, hipStream_t s)
+{
+    if (a.M > 32 || !tile_layout(a)) {
+        return false;
+    }
+    const TileArgs t = tile_args(a);
+    const int strips = (a.N + 15) / 16;
+    const dim3 grid(static_cast<unsigned>(strips));
+    if (a.M > 8) {
+        const int rounds = (strips + kTileCUs - 1) / kTileCUs;
+        const float rate = (a.M > 16 ? 2.3f : 1.5f) / 4096.f;
+        int shape;
+        if (3.4f + rate * static_cast<float>(rounds) * static_cast<float>(a.K) >
+            w4a8_tile_us(a, shape)) {
+            return false;
+        }
+    }
+    if (a.M > 16) {
+        hipLaunchKernelGGL((w4a8_skinny_kernel<8, 8, 1, OUT>), grid, dim3(512), 0, s, t);
+    } else if (strips > 2 * kTileCUs || a.K <= 2048) {
+        if (a.M <= 4) {
+            hipLaunchKernelGGL((w4a8_skinny_kernel<4, 1, 1, OUT>), grid, dim3(256), 0, s, t);
+        } else if (a.M <= 8) {
+            hipLaunchKernelGGL((w4a8_skinny_kernel<4, 2, 1, OUT>), grid, dim3(256), 0, s, t);
+        } else {
+            hipLaunchKernelGGL((w4a8_skinny_kernel<4, 4, 1, OUT>), grid, dim3(256), 0, s, t);
+        }
+    } else if (a.M <= 4) {
+        hipLaunchKernelGGL((w4a8_skinny_kernel<8, 1, 2, OUT>), grid, dim3(512), 0, s, t);
+    } else if (a.M <= 8) {
+        hipLaunchKernelGGL((w4a8_skinny_kernel<8, 2, 2, OUT>), grid, dim3(512), 0, s, t);
+    } else {
+        hipLaunchKernelGGL((w4a8_skinny_kernel<8, 4, 1, OUT>), grid, dim3(512), 0, s, t);
+    }
+    return true;
+}
+
+// The tile kernel for plain layouts whose rows are whole 32-k groups of aligned bytes; false when
+// it does not apply (the kernel's offsets are 32 bits from a tile's first row) or the k-split
+// kernel, if it does (`ksplit`), is the faster one.
+template <int OUT>
+bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
+{
+    if (!tile_layout(a)) {
+        return false;
+    }
+    TileArgs t = tile_args(a);
+    constexpr int kElem = OUT == OUT_F32 ? 4 : 2;
+    t.vec_d = a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.D) % (4 * kElem) == 0;
+    int best = 0;
+    const float best_us = w4a8_tile_us(a, best);
     const int passes = (a.M + kRowsPerChunk - 1) / kRowsPerChunk;
     if (ksplit && 3.2f + 0.115e-6f * static_cast<float>(a.N) * static_cast<float>(a.K) *
                               static_cast<float>(passes) <= best_us) {
@@ -933,6 +1000,8 @@ void w4a8_run(size_t m, size_t n, size_t k, const void *A, size_t lda, size_t k_
                       ldd < (1u << 24);
     if (fast && !packed && launch_w4a8_strip<OUT>(a, s)) {
         // decode strip kernel (m = 1, k = 2048 or 4096)
+    } else if (!packed && launch_w4a8_skinny<OUT>(a, s)) {
+        // few-row kernel
     } else if (!packed && launch_w4a8_tile<OUT>(a, fast, s)) {
         // large-tile kernel
     } else if (fast) {
