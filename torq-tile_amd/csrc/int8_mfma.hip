@@ -27,8 +27,9 @@
 //   * int8_mfma_kernel (igemmcl, the other 16-byte-aligned shapes, clamp_i32's [k, n] B): 256 threads
 //     (4 wave64s in a 2x2 grid) on a BM x 128 tile, k in steps of 64 bytes through double-buffered
 //     LDS tiles, v_mfma_i32_16x16x64_i8;
-//   * int8_generic_kernel: one thread per output for unaligned pointers or strides, k not a
-//     multiple of 16, or channel counts not a multiple of 16.
+//   * int8_edge_kernel (int8_edge.hpp): plain operands at any alignment, k and channel count;
+//   * int8_generic_kernel: one thread per output for what remains (a few outputs of a short k,
+//     packed, per-row quantized and channel-first operands that the others refuse).
 // All accumulate exactly in int32 and fuse the epilogue (C, bias, requantization,
 // saturation, clamp) into the store.
 #include <type_traits>
@@ -1991,6 +1992,7 @@ bool launch_small_clamp(const Int8Args &a, hipStream_t stream)
 #include "int8_skinny.hpp"
 #include "w8a8_tile.hpp"
 #include "conv_cf.hpp"
+#include "int8_edge.hpp"
 
 namespace tqt {
 namespace {
@@ -2042,6 +2044,12 @@ void launch_int8(const Int8Args &a, bool fast, hipStream_t stream, const char *w
     }
     if constexpr (AM == A_MATRIX && BMd == B_KN && EPI == EPI_CLAMP_I32 && PK == PK_NONE) {
         if (fast && a.d_row0 == 0 && launch_small_clamp(a, stream)) {
+            check_launch(where);
+            return;
+        }
+    }
+    if constexpr (PK == PK_NONE && BMd != B_CF && !is_dyn(EPI)) {
+        if (!fast && launch_edge<AM, BMd, EPI>(a, stream)) {
             check_launch(where);
             return;
         }
