@@ -1,4 +1,4 @@
-"""W4A16 few-row kernel (up to 16 rows): against exact f64 math and the CPU oracle at its row classes
+"""W4A16 few-row kernel (groups of up to 16 rows): against exact f64 math and the CPU oracle at its row classes
 (2, 8, 16), a ragged last strip of channels, k that leaves waves without a block or with part of one,
 both workgroup sizes, every block width class, odd scale strides, C, clamps and infinities."""
 
@@ -24,6 +24,9 @@ SHAPES = [
     (1, 8200, 544, 32),      # four waves a workgroup
     (5, 8197, 2304, 64),
     (16, 8193, 320, 64),
+    (17, 100, 2880, 96),     # two row groups, the second of one row
+    (33, 515, 4224, 64),
+    (64, 300, 11008, 128),
 ]
 
 

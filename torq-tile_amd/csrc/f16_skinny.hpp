@@ -1,7 +1,7 @@
-// Few-row f16 contraction with block-quantized int4 weights (W4A16 decode: up to 16 rows, every
-// scale block width that is a multiple of 32).
+// Few-row f16 contraction with block-quantized int4 weights (W4A16 decode and small prefill chunks:
+// groups of up to 16 rows, every scale block width that is a multiple of 32).
 //
-// A workgroup of WV wave64s owns 16 output channels over all of k; wave w takes the 256-k blocks w,
+// A workgroup of WV wave64s owns 16 output channels of one row group over all of k; wave w takes the 256-k blocks w,
 // w + WV, ... A block - 16 weight rows of 128 bytes (whole cache lines), the activation rows and the
 // scales of its eight 32-k sub-blocks - lands in a ring of the wave's own in LDS by direct global ->
 // LDS loads, is read into registers, and its slot refilled before the math. The waves meet once, at
@@ -13,7 +13,7 @@
 // terms; they and the waves' sums are added in f64 and rounded once.
 //
 // What bounds it: the weight stream behind a fixed 4 us (launch and the first loads' latency): 1 x
-// 28672 x 8192 (118 MB) runs at 3.8 TB/s, 34.5 us. The other kernels' fixed share is larger (they pad
+// 28672 x 8192 (118 MB) runs at 4.3 TB/s, 31 us. The other kernels' fixed share is larger (they pad
 // to 32 rows and meet all waves at each chunk of k), or they have too few workgroups. Before -> now:
 // 1 x 4096 x 4096 12.0 -> 6.5 us, 1 x 4096 x 14336 31.6 -> 12.0, 1 x 4096 x 11008 in 128-wide blocks
 // 37.3 -> 10.8, 8 x 4096 x 11008 41.7 -> 11.1, 16 x 4096 x 4096 12.3 -> 7.4.
@@ -33,8 +33,10 @@ struct F16SkinnyArgs
 };
 
 // XB: 1 KiB load blocks of activations per 256 k (two rows each); NS: blocks in flight per wave.
+// The register bound of the four-wave, two-row form lets four workgroups share a CU instead of three
+// (1 x 14336 x 4096, 3.5 workgroups a CU: 13.5 -> 12.1 us).
 template <int WV, int XB, int NS, int OUT>
-__global__ __launch_bounds__(WV * 64) void w4a16_skinny_kernel(F16SkinnyArgs fa)
+__global__ __launch_bounds__(WV * 64, WV == 4 && XB == 1 ? 4 : 2) void w4a16_skinny_kernel(F16SkinnyArgs fa)
 {
     const F16TileArgs &a = fa.t;
     constexpr int SW = 2048, SX = XB * 1024, SS = 512;
@@ -49,16 +51,18 @@ __global__ __launch_bounds__(WV * 64) void w4a16_skinny_kernel(F16SkinnyArgs fa)
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * 16;
+    const int m0 = blockIdx.y * 16;
+    const int rows = min(16, a.M - m0);
     const int fr = lane & 15;  // activation row / channel of the MFMA operands
     const int fg = lane >> 4;  // 8-k group
 
     // epilogue operands of this thread's output (the first 256: row tid / 16, channel tid % 16)
-    const int orow = (tid >> 4) & 15, gn = n0 + (tid & 15);
-    const int cn = min(gn, a.N - 1), cm = min(orow, a.M - 1);
+    const int orow = (tid >> 4) & 15, gm = m0 + orow, gn = n0 + (tid & 15);
+    const int cn = min(gn, a.N - 1), cm = min(gm, a.M - 1);
     const uint32_t p_bias = a.bias ? load_out_bits<OUT>(a.bias, cn) : 0u;
     const uint32_t p_c = a.C ? load_out_bits<OUT>(a.C, static_cast<long long>(cm) * a.ldc + cn) : 0u;
 
-    const i32x4 x_rsrc = raw_rsrc(a.A, kTileRecords);
+    const i32x4 x_rsrc = raw_rsrc(a.A + static_cast<long long>(m0) * a.lda, kTileRecords);
     const i32x4 w_rsrc = raw_rsrc(a.B + static_cast<long long>(n0) * a.bstride, kTileRecords);
     const uintptr_t s_addr =
         reinterpret_cast<uintptr_t>(a.scale_b + static_cast<long long>(n0) * a.ldsb);
@@ -83,7 +87,7 @@ __global__ __launch_bounds__(WV * 64) void w4a16_skinny_kernel(F16SkinnyArgs fa)
         const int row = 2 * j + (lane >> 5);
         const uint32_t chunk = static_cast<uint32_t>((lane & 31) ^ (row & 15));
         x_k[j] = chunk * 8;
-        x_off[j] = static_cast<uint32_t>(min(row, a.M - 1)) * static_cast<uint32_t>(2 * a.lda) +
+        x_off[j] = static_cast<uint32_t>(min(row, rows - 1)) * static_cast<uint32_t>(2 * a.lda) +
                    chunk * 16;
     }
     // scale index of 32-k block kb: kb / bdiv (kb < 2^17: exact by the rounded-up reciprocal)
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(WV * 64) void w4a16_skinny_kernel(F16SkinnyArgs fa)
         part[(4 * fg + r) * 16 + fr] = v;
     }
     __syncthreads();
-    if (tid >= 256 || orow >= a.M || gn >= a.N) {
+    if (tid >= 256 || gm >= a.M || gn >= a.N) {
         return;
     }
     double sum = 0.0;
@@ -210,7 +214,7 @@ __global__ __launch_bounds__(WV * 64) void w4a16_skinny_kernel(F16SkinnyArgs fa)
         v += out_from_bits<OUT>(p_bias);
     }
     const float cl = fminf(fmaxf(v, a.cmin), a.cmax);
-    store_out<OUT>(a.D, static_cast<long long>(orow) * a.ldd + gn,
+    store_out<OUT>(a.D, static_cast<long long>(gm) * a.ldd + gn,
                    v != v && !a.nan_to_min ? v : cl);
 }
 

@@ -748,18 +748,22 @@ bool tile_layout(const W4A16Args &a)
 }
 
 // Microseconds of the few-row kernel (f16_skinny.hpp), 0 where it does not apply: a fixed part and
-// the 16-channel strips that one CU streams one after another, more slowly with the activation rows
-// that each strip loads too. At k 4096 and one row: 256 strips 6.5, 512 8.7, 768 10.5, 896 13.5 (four
-// on some CUs); 1792 strips at k 8192 34.5; with 16 rows 7.4, 12.3, -, 17.7 and 48.5.
+// the 16-channel strips that one CU streams, more slowly with the activation rows that each strip
+// loads too. At k 4096 and one row: 256 strips 6.5, 512 8.7, 768 10.3, 896 12.1; 1792 strips at k 8192
+// 31; with 16 rows 7.4, 12.3, 13.0, 17.7 and 48.5. More than 16 rows, a group of 16 each, only where
+// the generic kernel is the alternative (26 x 1152 x 11008 in 128-wide blocks 11.7, 36.8 in tiles):
+// the 32-row kernels read the weights once.
 template <int OUT>
-float w4a16_skinny_us(const W4A16Args &a)
+float w4a16_skinny_us(const W4A16Args &a, bool listed)
 {
-    if (a.M > 16 || a.K < 128 || !tile_layout<OUT>(a)) {
+    if (a.M > (listed ? 16 : 64) || a.K < 128 || !tile_layout<OUT>(a)) {
         return 0.f;
     }
-    const int rounds = (a.ntiles + kTileCUs - 1) / kTileCUs;
-    return 4.3f + 2.15f / 4096.f * static_cast<float>(rounds) * static_cast<float>(a.K) *
-                      (1.f + 0.0022f * static_cast<float>(a.M * a.M));
+    const long long strips = static_cast<long long>(a.ntiles) * ((a.M + 15) / 16);
+    const long long rounds = (strips + kTileCUs - 1) / kTileCUs;
+    const int rows = a.M < 16 ? a.M : 16;
+    return 4.2f + 1.95f / 4096.f * static_cast<float>(rounds) * static_cast<float>(a.K) *
+                      (1.f + 0.0027f * static_cast<float>(rows * rows));
 }
 
 template <int OUT>
@@ -768,11 +772,12 @@ void launch_w4a16_skinny(const W4A16Args &a, bool nan_to_min, hipStream_t s)
     F16SkinnyArgs f = {};
     f.t = tile_args(a, nan_to_min);
     f.bdiv = static_cast<uint32_t>(a.bl / 32);
-    const dim3 grid(static_cast<unsigned>(a.ntiles));
-    // More than two strips a CU: half the waves and one block in flight each, so that four are
-    // resident together (1 x 14336 x 4096: 13.5 us, 14.1 with eight waves; 1 x 4096 x 4096: 7.2 and
-    // 6.6).
-    if (a.ntiles > 2 * kTileCUs) {
+    const int groups = (a.M + 15) / 16;
+    const dim3 grid(static_cast<unsigned>(a.ntiles), static_cast<unsigned>(groups));
+    // More than two strips a CU: half the waves and one block in flight each, so that with few rows
+    // four are resident together (1 x 14336 x 4096: 12.1 us, 14.1 with eight waves; 1 x 4096 x 4096:
+    // 7.2 and 6.6).
+    if (static_cast<long long>(a.ntiles) * groups > 2 * kTileCUs) {
         const dim3 block(256);
         if (a.M <= 2) {
             hipLaunchKernelGGL((w4a16_skinny_kernel<4, 1, 1, OUT>), grid, block, 0, s, f);
@@ -920,9 +925,10 @@ void w4a16_run(size_t m, size_t n, size_t k, size_t bl, const void *A, size_t ld
                    (3.5f + static_cast<float>(a.K) * (0.002f + 0.0006f * strip));
     }
     const F16TilePick tile = packed ? F16TilePick{0.f, 0, 0} : w4a16_tile_pick<OUT>(a, other_us);
-    const float skinny_us = packed ? 0.f : w4a16_skinny_us<OUT>(a);
     const bool listed = other_us > 0.f;
-    if (skinny_us > 0.f && (!listed || skinny_us < other_us) &&
+    const float skinny_us = packed ? 0.f : w4a16_skinny_us<OUT>(a, listed);
+    // (other_us reads about a tenth low against it: 1 x 14336 x 4096 11.3, measured 13.0)
+    if (skinny_us > 0.f && (!listed || skinny_us < 1.1f * other_us) &&
         (tile.us == 0.f || skinny_us < tile.us)) {
         launch_w4a16_skinny<OUT>(a, listed, s);
     } else if (tile.us > 0.f && (!listed || tile.us < other_us)) {

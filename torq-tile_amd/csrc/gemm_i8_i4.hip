@@ -825,21 +825,26 @@ inline float w4a8_tile_us(const W4A8Args &a, int &best)
 
 // Few rows (int4_skinny.hpp); false where it does not apply or is the slower one. Measured on
 // MI355X (us, weights partly cached; the k-split or tile kernel in parentheses): up to 8 rows it
-// wins at every size - 8 x 4096 x 11008 7.4 (8.1), 4 x 896 x 13792 5.9 (30.8), 8 x 28672 x 8192 22.5
-// (23.1). With more rows the activations weigh as much as the weights and each 16-channel strip
-// reloads them: 9 x 5120 x 12544 10.7 (15.1), 16 x 11008 x 4096 6.9 (12.3), 16 x 28672 x 8192 26.7
-// (24), 32 x 4096 x 4096 5.8 (8.0), 32 x 11008 x 4096 11.1 (12.7), 32 x 28672 x 8192 35 (24).
+// wins - 8 x 4096 x 11008 7.4 (8.1), 4 x 896 x 13792 5.9 (30.8), 8 x 28672 x 8192 22.5 (23.1) - but
+// where the k-split kernel applies and gives each wave one or two loads (k over 2048, to 4096) on
+// a strip or two a CU: 8 x 4096 x 4096 4.8 (4.5), 2 x 1280 x 3840 3.7 (3.5). With more rows the
+// activations weigh as much as the weights and each 16-channel strip reloads them: 9 x 5120 x 12544
+// 10.7 (15.1), 16 x 11008 x 4096 6.9 (12.3), 16 x 28672 x 8192 26.7 (24), 32 x 4096 x 4096 5.8
+// (8.0), 32 x 11008 x 4096 11.1 (12.7), 32 x 28672 x 8192 35 (24).
 // Four waves a workgroup where a CU gets more than two strips (16 x 11008 x 4096 6.9, 8.4 with
 // eight) or k leaves eight little to do (1 x 5504 x 1024 3.2, 4.0); eight stream one strip faster
 // (4 x 896 x 13792 5.9, 8.4 with four).
 template <int OUT>
-bool launch_w4a8_skinny(const W4A8Args &a, hipStream_t s)
+bool launch_w4a8_skinny(const W4A8Args &a, bool ksplit, hipStream_t s)
 {
     if (a.M > 32 || !tile_layout(a)) {
         return false;
     }
-    const TileArgs t = tile_args(a);
     const int strips = (a.N + 15) / 16;
+    if (ksplit && a.M <= 8 && a.K > 2048 && a.K <= 4096 && strips <= 2 * kTileCUs) {
+        return false;
+    }
+    const TileArgs t = tile_args(a);
     const dim3 grid(static_cast<unsigned>(strips));
     if (a.M > 8) {
         const int rounds = (strips + kTileCUs - 1) / kTileCUs;
@@ -1000,7 +1005,7 @@ void w4a8_run(size_t m, size_t n, size_t k, const void *A, size_t lda, size_t k_
                       ldd < (1u << 24);
     if (fast && !packed && launch_w4a8_strip<OUT>(a, s)) {
         // decode strip kernel (m = 1, k = 2048 or 4096)
-    } else if (!packed && launch_w4a8_skinny<OUT>(a, s)) {
+    } else if (!packed && launch_w4a8_skinny<OUT>(a, fast, s)) {
         // few-row kernel
     } else if (!packed && launch_w4a8_tile<OUT>(a, fast, s)) {
         // large-tile kernel
