@@ -1,0 +1,31 @@
+// The dispatch rules of torq-tile_amd/csrc/route.hpp behind C symbols, for the host tests.
+#include "route.hpp"
+
+using namespace tqt;
+
+extern "C" {
+
+uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
+{
+    return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));
+}
+
+int tqtr_w4a16_skinny_scales_exact(long long k, long long bl)
+{
+    return w4a16_skinny_scales_exact(k, bl);
+}
+
+// The first 32-k block of k whose scale block the reciprocal gets wrong, or -1.
+long long tqtr_first_wrong_scale_block(long long k, long long bl)
+{
+    const uint32_t bdiv = static_cast<uint32_t>(bl / 32);
+    const uint32_t inv = scale_block_inverse(bdiv);
+    for (long long kb = 0; kb < k / 32; ++kb) {
+        if (scale_block_of(static_cast<uint32_t>(kb), bdiv, inv) != kb / bdiv) {
+            return kb;
+        }
+    }
+    return -1;
+}
+
+}  // extern "C"

@@ -61,3 +61,25 @@ def test_w4a16_skinny_infinity(gpu, n):
         assert np.isnan(got[row, q == 0]).all()
         assert (got[row, q > 0] == sign * np.inf).all() and (got[row, q < 0] == -sign * np.inf).all()
     assert np.isfinite(got[[0, 1, 3, 4]]).all()
+
+
+@pytest.mark.parametrize("k,bl", [(2097184, 2097184), (3 * 1213664, 1213664)])
+def test_w4a16_very_wide_blocks(gpu, k, bl):
+    """Scale blocks past the few-row kernel's exact indexes (bl / 32 * k / 32 > 2^32): the last 32 k
+    count. Only they are not zero, so that the sums are short ones."""
+    m, n = 2, 18
+    rng = np.random.default_rng(3)
+    A = np.zeros((m, k), np.float16)
+    A[:, -32:] = rng.standard_normal((m, 32))
+    Bp = np.full((n, k // 2), 0x88, np.uint8)
+    Bp[:, -16:] = rng.integers(0, 256, (n, 16))
+    S = rng.uniform(0.005, 0.02, (n, k // bl)).astype(np.float16)
+    d = dict(A16=A.view(np.uint16), Bp=Bp, S16=S.view(np.uint16), bl=bl, C16=None, bias16=None)
+    got = _run_f32(d)
+    q = np.empty((n, 32))
+    q[:, 0::2] = (Bp[:, -16:] & 15).astype(np.float64) - 8
+    q[:, 1::2] = (Bp[:, -16:] >> 4).astype(np.float64) - 8
+    w = q * S[:, -1:].astype(np.float64)
+    a = A[:, -32:].astype(np.float64)
+    # 32 products and their sum, the scale, and three additions of zero: 64 roundings at most
+    assert (np.abs(got - a @ w.T) <= 64 * 2.0 ** -24 * (np.abs(a) @ np.abs(w).T)).all()

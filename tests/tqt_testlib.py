@@ -15,6 +15,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ORACLE_SO = os.path.join(ROOT, "oracle", "liboracle.so")
 REF_SO = os.path.join(ROOT, "oracle", "_ref", "libtqt_ref.so")
 SHIM_SO = os.path.join(ROOT, "tests", "abi_shim", "libtqt_test_shim.so")
+ROUTE_SO = os.path.join(ROOT, "tests", "abi_shim", "libtqt_route_shim.so")
 GOLDEN_DIR = os.path.join(ROOT, "tests", "golden")
 
 c_size = ctypes.c_size_t

@@ -20,6 +20,7 @@
 #pragma once
 
 #include "f16_tile.hpp"
+#include "route.hpp"
 
 namespace tqt {
 namespace {
@@ -90,9 +91,10 @@ __global__ __launch_bounds__(WV * 64, WV == 4 && XB == 1 ? 4 : 2) void w4a16_ski
         x_off[j] = static_cast<uint32_t>(min(row, rows - 1)) * static_cast<uint32_t>(2 * a.lda) +
                    chunk * 16;
     }
-    // scale index of 32-k block kb: kb / bdiv (kb < 2^17: exact by the rounded-up reciprocal)
-    const uint32_t inv = static_cast<uint32_t>((0x100000000ull + fa.bdiv - 1) / fa.bdiv);
-    auto scale_idx = [&](uint32_t kb) { return fa.bdiv == 1 ? kb : __umulhi(kb, inv); };
+    // scale index of 32-k block kb (the launcher keeps k and the block width where it is exact; past
+    // the last block it may only read high, and is refused by its count all the same)
+    const uint32_t inv = scale_block_inverse(fa.bdiv);
+    auto scale_idx = [&](uint32_t kb) { return scale_block_of(kb, fa.bdiv, inv); };
     int8_t *mine = ring + wave * RING;
     const uint32_t K = static_cast<uint32_t>(a.K);
     auto issue = [&](int it, int slot) {

@@ -736,14 +736,15 @@ inline F16TileArgs tile_args(const W4A16Args &a, bool nan_to_min)
     return t;
 }
 
-// Layouts the tile kernels take: 16-byte aligned rows, scale blocks of whole 32-k groups, strides
-// within their 32-bit offsets.
+// Layouts the tile kernels take: 16-byte aligned rows, scale blocks of whole 32-k groups, strides and
+// k (a single row's stride bounds nothing) within their 32-bit offsets.
 template <int OUT>
 bool tile_layout(const W4A16Args &a)
 {
     constexpr long long kElem = OUT == OUT_F32 ? 4 : 2;
-    return a.K > 0 && a.bl % 32 == 0 && a.lda % 8 == 0 && a.bstride % 16 == 0 && aligned16(a.A) &&
-           aligned16(a.B) && a.lda < (1 << 22) && a.bstride < (1 << 22) && a.ldsb < (1 << 22) &&
+    return a.K > 0 && a.K < (1 << 22) && a.bl % 32 == 0 && a.lda % 8 == 0 &&
+           a.bstride % 16 == 0 && aligned16(a.A) && aligned16(a.B) &&
+           a.lda < (1 << 22) && a.bstride < (1 << 22) && a.ldsb < (1 << 22) &&
            a.ldd * kElem < (1 << 23) && (!a.C || a.ldc * kElem < (1 << 23));
 }
 
@@ -756,7 +757,8 @@ bool tile_layout(const W4A16Args &a)
 template <int OUT>
 float w4a16_skinny_us(const W4A16Args &a, bool listed)
 {
-    if (a.M > (listed ? 16 : 64) || a.K < 128 || !tile_layout<OUT>(a)) {
+    if (a.M > (listed ? 16 : 64) || a.K < 128 || !tile_layout<OUT>(a) ||
+        !w4a16_skinny_scales_exact(a.K, a.bl)) {
         return 0.f;
     }
     const long long strips = static_cast<long long>(a.ntiles) * ((a.M + 15) / 16);
