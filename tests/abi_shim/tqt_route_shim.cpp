@@ -5,6 +5,11 @@ using namespace tqt;
 
 extern "C" {
 
+int tqtr_grid_fits(long long blocks, int threads)
+{
+    return grid_fits(blocks, threads);
+}
+
 uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
 {
     return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));

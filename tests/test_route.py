@@ -35,3 +35,10 @@ def test_wide_scale_blocks_refused(rules, k, bl):
     kernels."""
     assert rules.tqtr_first_wrong_scale_block(k, bl) >= 0
     assert not rules.tqtr_w4a16_skinny_scales_exact(k, bl)
+
+
+def test_grid_fits(rules):
+    """A grid dimension holds fewer than 2^32 work-items."""
+    rules.tqtr_grid_fits.argtypes = [ctypes.c_longlong, ctypes.c_int]
+    assert rules.tqtr_grid_fits((1 << 23) - 1, 512) and not rules.tqtr_grid_fits(1 << 23, 512)
+    assert rules.tqtr_grid_fits((1 << 24) - 1, 256) and not rules.tqtr_grid_fits(1 << 24, 256)

@@ -294,7 +294,7 @@ inline bool launch_conv_cf(const Int8Args &a, hipStream_t stream)
     hp.px_rows = static_cast<int>(rows);
     hp.tiles_c = (a.M + kCfCh - 1) / kCfCh;
     const long long tiles = static_cast<long long>((a.N + kCfPix - 1) / kCfPix) * hp.tiles_c;
-    if (tiles >= (1ll << 28)) {
+    if (!grid_fits(tiles + 8, 256)) {
         return false;
     }
     hp.tiles = static_cast<int>(tiles);

@@ -20,7 +20,6 @@
 #pragma once
 
 #include "f16_tile.hpp"
-#include "route.hpp"
 
 namespace tqt {
 namespace {

@@ -646,21 +646,21 @@ int device_cu_count()
 // ---------------------------------------------------------------------------------------------
 struct F16TileShape
 {
-    int bm, bn;
+    int bm, bn, threads;
     float fixed, stage;            // us of one round
     float pair_fixed, pair_stage;  // us of two
 };
 constexpr int kF16Shapes = 4;
 constexpr F16TileShape kF16Tiles[3][kF16Shapes] = {
     // 32-wide blocks
-    {{128, 256, 9.f, 3.1f, 18.f, 6.2f}, {128, 128, 6.f, 1.6f, 12.f, 3.2f},
-     {64, 128, 4.5f, .95f, 5.f, 1.85f}, {32, 64, 4.2f, .44f, 5.f, .61f}},
+    {{128, 256, 512, 9.f, 3.1f, 18.f, 6.2f}, {128, 128, 512, 6.f, 1.6f, 12.f, 3.2f},
+     {64, 128, 256, 4.5f, .95f, 5.f, 1.85f}, {32, 64, 256, 4.2f, .44f, 5.f, .61f}},
     // blocks of a multiple of 64
-    {{128, 256, 9.f, 2.2f, 18.f, 4.4f}, {128, 128, 6.f, 1.4f, 12.f, 2.8f},
-     {64, 128, 4.5f, .9f, 5.f, 1.45f}, {32, 64, 4.2f, .38f, 5.f, .58f}},
+    {{128, 256, 512, 9.f, 2.2f, 18.f, 4.4f}, {128, 128, 512, 6.f, 1.4f, 12.f, 2.8f},
+     {64, 128, 256, 4.5f, .9f, 5.f, 1.45f}, {32, 64, 256, 4.2f, .38f, 5.f, .58f}},
     // compensated: the registers of the two larger tiles do not suffice
-    {{0, 0, 0.f, 0.f, 0.f, 0.f}, {0, 0, 0.f, 0.f, 0.f, 0.f},
-     {64, 128, 4.5f, 1.4f, 5.f, 2.6f}, {32, 64, 4.2f, .57f, 5.f, .8f}}};
+    {{0, 0, 0, 0.f, 0.f, 0.f, 0.f}, {0, 0, 0, 0.f, 0.f, 0.f, 0.f},
+     {64, 128, 256, 4.5f, 1.4f, 5.f, 2.6f}, {32, 64, 256, 4.2f, .57f, 5.f, .8f}}};
 
 template <int MI, int WGN, int KS, int NS, int SPB, int COMP, int OUT>
 void launch_f16_tile(F16TileArgs t, hipStream_t s)
@@ -668,8 +668,7 @@ void launch_f16_tile(F16TileArgs t, hipStream_t s)
     constexpr int BM = 32 * MI, BN = 32 * WGN;
     t.tiles_m = (t.M + BM - 1) / BM;
     t.tiles_n = (t.N + BN - 1) / BN;
-    const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;
-    TQT_REQUIRE(tiles < (1ll << 28), "grid too large");
+    const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;  // (the pick bounds them)
     t.per_xcd = static_cast<int>((tiles + 7) / 8);
     hipLaunchKernelGGL((w4a16_tile_kernel<MI, WGN, KS, NS, SPB, COMP, OUT>),
                        dim3(8 * static_cast<unsigned>(t.per_xcd)), dim3(64 * WGN * KS), 0, s, t);
@@ -762,6 +761,9 @@ float w4a16_skinny_us(const W4A16Args &a, bool listed)
         return 0.f;
     }
     const long long strips = static_cast<long long>(a.ntiles) * ((a.M + 15) / 16);
+    if (!grid_fits(a.ntiles, 512)) {
+        return 0.f;
+    }
     const long long rounds = (strips + kTileCUs - 1) / kTileCUs;
     const int rows = a.M < 16 ? a.M : 16;
     return 4.2f + 1.95f / 4096.f * static_cast<float>(rounds) * static_cast<float>(a.K) *
@@ -829,6 +831,9 @@ F16TilePick w4a16_tile_pick(const W4A16Args &a, float other_us)
         const F16TileShape &p = kF16Tiles[best.variant][i];
         const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
                                 ((a.N + p.bn - 1) / p.bn);
+        if (!grid_fits(tiles + 8, p.threads)) {
+            continue;
+        }
         const long long rounds = (tiles + kTileCUs - 1) / kTileCUs;
         const float us =
             static_cast<float>(rounds / 2) * (p.pair_fixed + p.pair_stage * stages) +

@@ -754,11 +754,14 @@ bool launch_w4a8_qstrip(const W4A8Args &a, const float *X, int8_t *Aq, float *sa
 // ---------------------------------------------------------------------------------------------
 struct TileShape
 {
-    int bm, bn;
+    int bm, bn, threads;
     float fixed, stage;  // us per round: fixed + stage * ceil(k / 128)
 };
 constexpr TileShape kTileShapes[] = {
-    {256, 256, 18.0f, 2.0f}, {128, 128, 5.0f, 0.57f}, {64, 128, 4.5f, 0.32f}, {32, 128, 4.0f, 0.24f}};
+    {256, 256, 512, 18.0f, 2.0f},
+    {128, 128, 256, 5.0f, 0.57f},
+    {64, 128, 256, 4.5f, 0.32f},
+    {32, 128, 256, 4.0f, 0.24f}};
 
 template <int MI, int NI, int WGM, int WGN, int KS, int NS, int OUT>
 void launch_tile(TileArgs t, hipStream_t s)
@@ -767,7 +770,6 @@ void launch_tile(TileArgs t, hipStream_t s)
     t.tiles_m = (t.M + BM - 1) / BM;
     t.tiles_n = (t.N + BN - 1) / BN;
     const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;
-    TQT_REQUIRE(tiles < (1ll << 28), "grid too large");
     t.per_xcd = static_cast<int>((tiles + 7) / 8);
     hipLaunchKernelGGL((w4a8_tile_kernel<MI, NI, WGM, WGN, KS, NS, OUT>),
                        dim3(8 * static_cast<unsigned>(t.per_xcd)), dim3(64 * WGM * WGN * KS), 0, s, t);
@@ -804,7 +806,7 @@ inline bool tile_layout(const W4A8Args &a)
            aligned16(a.A) && aligned16(a.B) && a.lda < (1 << 22) && a.bstride < (1 << 22);
 }
 
-// Microseconds of the cheapest tile shape, and which it is.
+// Microseconds of the cheapest tile shape, and which it is; 0 where no shape's grid fits.
 inline float w4a8_tile_us(const W4A8Args &a, int &best)
 {
     const float stages = static_cast<float>((a.K + kTileK - 1) / kTileK);
@@ -813,9 +815,12 @@ inline float w4a8_tile_us(const W4A8Args &a, int &best)
         const TileShape &p = kTileShapes[i];
         const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
                                 ((a.N + p.bn - 1) / p.bn);
+        if (!grid_fits(tiles + 8, p.threads)) {
+            continue;
+        }
         const float us = static_cast<float>((tiles + kTileCUs - 1) / kTileCUs) *
                          (p.fixed + p.stage * stages);
-        if (i == 0 || us < best_us) {
+        if (best_us == 0.f || us < best_us) {
             best = i;
             best_us = us;
         }
@@ -841,6 +846,9 @@ bool launch_w4a8_skinny(const W4A8Args &a, bool ksplit, hipStream_t s)
         return false;
     }
     const int strips = (a.N + 15) / 16;
+    if (!grid_fits(strips, 512)) {
+        return false;
+    }
     if (ksplit && a.M <= 8 && a.K > 2048 && a.K <= 4096 && strips <= 2 * kTileCUs) {
         return false;
     }
@@ -889,6 +897,9 @@ bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
     t.vec_d = a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.D) % (4 * kElem) == 0;
     int best = 0;
     const float best_us = w4a8_tile_us(a, best);
+    if (best_us == 0.f) {
+        return false;
+    }
     const int passes = (a.M + kRowsPerChunk - 1) / kRowsPerChunk;
     if (ksplit && 3.2f + 0.115e-6f * static_cast<float>(a.N) * static_cast<float>(a.K) *
                               static_cast<float>(passes) <= best_us) {

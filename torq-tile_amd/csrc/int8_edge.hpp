@@ -260,7 +260,7 @@ bool launch_edge(const Int8Args &a, hipStream_t stream)
     }
     const long long blocks = static_cast<long long>((a.M + kEdgeT - 1) / kEdgeT) *
                              ((a.N + kEdgeT - 1) / kEdgeT);
-    if (blocks >= (1ll << 31)) {
+    if (!grid_fits(blocks, 256)) {
         return false;
     }
     hipLaunchKernelGGL((int8_edge_kernel<AM, BMd, EPI>), dim3(static_cast<unsigned>(blocks)),

@@ -254,7 +254,7 @@ template <int EPI, int PK>
 bool launch_skinny(const Int8Args &a, hipStream_t stream)
 {
     const int passes = (a.M + 31) / 32;
-    if (passes > 4 || a.K == 0 || a.lda >= (1 << 22) || a.ldb >= (1 << 22)) {
+    if (!grid_fits((a.N + kSkinnyN - 1) / kSkinnyN, 64 * kSkinnyWaves) || passes > 4 || a.K == 0 || a.lda >= (1 << 22) || a.ldb >= (1 << 22)) {
         return false;
     }
     if (passes > 1) {

@@ -43,6 +43,7 @@
 
 #include <type_traits>
 
+#include "route.hpp"
 #include "tqt_hip_common.hpp"
 
 namespace tqt {
@@ -55,7 +56,6 @@ __host__ __device__ constexpr int tile_waitcnt(int vm)
     return (vm & 15) | (7 << 4) | ((vm >> 4) << 14);
 }
 
-constexpr int kTileCUs = 256;                // compute units of an MI355X
 constexpr int kTileK = 128;                  // k per stage
 constexpr int kTileRingBytes = 150 * 1024;   // LDS for the ring, at most
 constexpr uint32_t kTileOob = 0x80000000u;   // a buffer offset past every resource below

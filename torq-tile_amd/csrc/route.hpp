@@ -6,6 +6,15 @@
 
 namespace tqt {
 
+constexpr int kTileCUs = 256;  // compute units of an MI355X
+
+// Whether `blocks` workgroups of `threads` fit one grid dimension: a launch counts its work-items along
+// a dimension in 32 bits.
+constexpr bool grid_fits(long long blocks, int threads)
+{
+    return blocks * threads < 0x100000000ll;
+}
+
 // ---------------------------------------------------------------------------------------------
 // W4A16
 // ---------------------------------------------------------------------------------------------

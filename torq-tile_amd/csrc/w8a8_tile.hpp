@@ -410,7 +410,6 @@ void launch_w8_tile(const Int8Args &a, hipStream_t stream)
     constexpr int BM = 32 * MI * WGM, BN = 32 * NI * WGN;
     const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
     const long long tiles = static_cast<long long>(tiles_m) * tiles_n;
-    TQT_REQUIRE(tiles < (1ll << 28), "grid too large");
     const int per_xcd = static_cast<int>((tiles + 7) / 8);
     constexpr int kVec = EPI == EPI_REQUANT_I8 ? 16 : 4;
     constexpr int kElem = EPI == EPI_REQUANT_I8 ? 1 : (EPI == EPI_DYN_F32 ? 4 : 2);
@@ -455,9 +454,11 @@ bool launch_w8a8_tile(const Int8Args &a, hipStream_t stream)
     const float mid_us =
         static_cast<float>(r128 / 2) * (kDyn ? 6.f + 1.5f * n : 5.f + 1.2f * n) +
         static_cast<float>(r128 % 2) * (kDyn ? 6.f + 0.9f * n : 4.f + 0.7f * n);
+    const long long t256 = static_cast<long long>((a.M + 255) / 256) * ((a.N + 255) / 256);
     const float big_us = static_cast<float>(r256) * (kDyn ? 20.f + 1.8f * n : 14.f + 1.5f * n);
     const long long t128 = static_cast<long long>((a.M + 127) / 128) * ((a.N + 127) / 128);
-    if (t128 <= (other ? 3 * kTileCUs / 4 : kTileCUs) || (stream_us <= mid_us && stream_us <= big_us)) {
+    if (!grid_fits(t256 + 8, 512) || !grid_fits(t128 + 8, 256) ||
+        t128 <= (other ? 3 * kTileCUs / 4 : kTileCUs) || (stream_us <= mid_us && stream_us <= big_us)) {
         return false;
     }
     if (big_us < mid_us) {
