@@ -10,6 +10,11 @@ int tqtr_grid_fits(long long blocks, int threads)
     return grid_fits(blocks, threads);
 }
 
+int tqtr_w4a8_route(long long m, long long n, long long k, int ksplit)
+{
+    return w4a8_route(m, n, k, ksplit != 0);
+}
+
 uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
 {
     return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));

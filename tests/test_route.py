@@ -4,6 +4,8 @@ import ctypes
 
 import pytest
 
+import tqt_testlib as T
+
 
 @pytest.fixture()
 def rules(route):
@@ -11,6 +13,7 @@ def rules(route):
     route.tqtr_first_wrong_scale_block.restype = ctypes.c_longlong
     route.tqtr_first_wrong_scale_block.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
     route.tqtr_w4a16_skinny_scales_exact.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
+    route.tqtr_w4a8_route.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     return route
 
 
@@ -42,3 +45,23 @@ def test_grid_fits(rules):
     rules.tqtr_grid_fits.argtypes = [ctypes.c_longlong, ctypes.c_int]
     assert rules.tqtr_grid_fits((1 << 23) - 1, 512) and not rules.tqtr_grid_fits(1 << 23, 512)
     assert rules.tqtr_grid_fits((1 << 24) - 1, 256) and not rules.tqtr_grid_fits(1 << 24, 256)
+
+
+# (m, n, k, whether the k-split kernel was the faster one): each from a side-by-side measurement with
+# the weights from HBM, where the two differ by 5% and more
+@pytest.mark.parametrize("m,n,k,ksplit", [
+    (1, 8192, 8192, True), (2, 8192, 8192, True), (8, 8192, 8192, True), (1, 5120, 13824, True),
+    (2, 11008, 4096, True), (2, 6272, 2816, True), (8, 4096, 4096, True), (1, 25216, 8448, True),
+    (1, 26176, 5888, True), (9, 8192, 8192, True), (17, 1280, 3840, True), (24, 2048, 2048, True),
+    (17, 512, 2048, True), (2, 2048, 2048, True), (1, 272, 4608, True),
+    (2, 16384, 512, False), (4, 1024, 1024, False), (1, 896, 13824, False), (8, 896, 13824, False),
+    (8, 4096, 11008, False), (8, 5120, 13824, False), (8, 17648, 9472, False),
+    (4, 9008, 11264, False), (8, 12080, 4608, False), (2, 18720, 1792, False),
+    (8, 15712, 3072, False), (12, 6352, 4608, False),
+    (16, 4096, 4096, False), (32, 4096, 4096, False), (32, 7616, 1280, False),
+])
+def test_w4a8_few_rows(rules, m, n, k, ksplit):
+    want = T.W4A8_OTHER if ksplit else T.W4A8_FEW_ROW
+    assert rules.tqtr_w4a8_route(m, n, k, 1) == want
+    # off the 256 grid of k the few-row kernel has only the tiles beside it
+    assert rules.tqtr_w4a8_route(m, n, k + 32, 0) != T.W4A8_OTHER

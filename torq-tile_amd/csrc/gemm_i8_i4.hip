@@ -740,29 +740,7 @@ bool launch_w4a8_qstrip(const W4A8Args &a, const float *X, int8_t *Aq, float *sa
     return true;
 }
 
-// ---------------------------------------------------------------------------------------------
-// Large-tile kernel (int8_tile.hpp): which tile a shape takes. Every tile is one pass of a CU over
-// k, so the launch costs ceil(tiles / 256) times (fixed + stages * rate) of its tile; the rates
-// below are microseconds measured on MI355X at k 864 and 4096 (M x N tiles: 256 x 256 82 us for
-// one round of 256 at k 4096, 128 x 128 23, 64 x 128 14.7, 32 x 128 11.7), and the cheapest wins:
-// 1000 x 11008 x 4096 takes 128 x 128 tiles (69 us; 74 with 256 x 256, 79 with 64 x 128, 108 with
-// 32 x 128), 512 x 4096 x 4096 64 x 128 (18.3; 25.7, 21.6 with 32 x 128), 4096^3 256 x 256 (82; 97).
-// The k-split kernel above, where it applies, costs one pass over the weights per 15 rows instead:
-// 3.2 us + 0.115 us per 10^6 weights and pass (11008 x 4096: 8.1 us at 12 rows, 12.6 at 16, 18.5 at
-// 32, 23.0 at 48, against 12.2-12.8 for the tiles; 4096 x 4096: 9.7 at 48 and 27.1 at 200, against
-// 12.5 and 12.8).
-// ---------------------------------------------------------------------------------------------
-struct TileShape
-{
-    int bm, bn, threads;
-    float fixed, stage;  // us per round: fixed + stage * ceil(k / 128)
-};
-constexpr TileShape kTileShapes[] = {
-    {256, 256, 512, 18.0f, 2.0f},
-    {128, 128, 256, 5.0f, 0.57f},
-    {64, 128, 256, 4.5f, 0.32f},
-    {32, 128, 256, 4.0f, 0.24f}};
-
+// Large-tile and few-row kernels (int8_tile.hpp, int4_skinny.hpp); which takes a shape: route.hpp.
 template <int MI, int NI, int WGM, int WGN, int KS, int NS, int OUT>
 void launch_tile(TileArgs t, hipStream_t s)
 {
@@ -806,63 +784,15 @@ inline bool tile_layout(const W4A8Args &a)
            aligned16(a.A) && aligned16(a.B) && a.lda < (1 << 22) && a.bstride < (1 << 22);
 }
 
-// Microseconds of the cheapest tile shape, and which it is; 0 where no shape's grid fits.
-inline float w4a8_tile_us(const W4A8Args &a, int &best)
-{
-    const float stages = static_cast<float>((a.K + kTileK - 1) / kTileK);
-    float best_us = 0.f;
-    for (int i = 0; i < 4; ++i) {
-        const TileShape &p = kTileShapes[i];
-        const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
-                                ((a.N + p.bn - 1) / p.bn);
-        if (!grid_fits(tiles + 8, p.threads)) {
-            continue;
-        }
-        const float us = static_cast<float>((tiles + kTileCUs - 1) / kTileCUs) *
-                         (p.fixed + p.stage * stages);
-        if (best_us == 0.f || us < best_us) {
-            best = i;
-            best_us = us;
-        }
-    }
-    return best_us;
-}
-
-// Few rows (int4_skinny.hpp); false where it does not apply or is the slower one. Measured on
-// MI355X (us, weights partly cached; the k-split or tile kernel in parentheses): up to 8 rows it
-// wins - 8 x 4096 x 11008 7.4 (8.1), 4 x 896 x 13792 5.9 (30.8), 8 x 28672 x 8192 22.5 (23.1) - but
-// where the k-split kernel applies and gives each wave one or two loads (k over 2048, to 4096) on
-// a strip or two a CU: 8 x 4096 x 4096 4.8 (4.5), 2 x 1280 x 3840 3.7 (3.5). With more rows the
-// activations weigh as much as the weights and each 16-channel strip reloads them: 9 x 5120 x 12544
-// 10.7 (15.1), 16 x 11008 x 4096 6.9 (12.3), 16 x 28672 x 8192 26.7 (24), 32 x 4096 x 4096 5.8
-// (8.0), 32 x 11008 x 4096 11.1 (12.7), 32 x 28672 x 8192 35 (24).
 // Four waves a workgroup where a CU gets more than two strips (16 x 11008 x 4096 6.9, 8.4 with
 // eight) or k leaves eight little to do (1 x 5504 x 1024 3.2, 4.0); eight stream one strip faster
 // (4 x 896 x 13792 5.9, 8.4 with four).
 template <int OUT>
-bool launch_w4a8_skinny(const W4A8Args &a, bool ksplit, hipStream_t s)
+void launch_w4a8_skinny(const W4A8Args &a, hipStream_t s)
 {
-    if (a.M > 32 || !tile_layout(a)) {
-        return false;
-    }
     const int strips = (a.N + 15) / 16;
-    if (!grid_fits(strips, 512)) {
-        return false;
-    }
-    if (ksplit && a.M <= 8 && a.K > 2048 && a.K <= 4096 && strips <= 2 * kTileCUs) {
-        return false;
-    }
     const TileArgs t = tile_args(a);
     const dim3 grid(static_cast<unsigned>(strips));
-    if (a.M > 8) {
-        const int rounds = (strips + kTileCUs - 1) / kTileCUs;
-        const float rate = (a.M > 16 ? 2.3f : 1.5f) / 4096.f;
-        int shape;
-        if (3.4f + rate * static_cast<float>(rounds) * static_cast<float>(a.K) >
-            w4a8_tile_us(a, shape)) {
-            return false;
-        }
-    }
     if (a.M > 16) {
         hipLaunchKernelGGL((w4a8_skinny_kernel<8, 8, 1, OUT>), grid, dim3(512), 0, s, t);
     } else if (strips > 2 * kTileCUs || a.K <= 2048) {
@@ -880,38 +810,20 @@ bool launch_w4a8_skinny(const W4A8Args &a, bool ksplit, hipStream_t s)
     } else {
         hipLaunchKernelGGL((w4a8_skinny_kernel<8, 4, 1, OUT>), grid, dim3(512), 0, s, t);
     }
-    return true;
 }
 
-// The tile kernel for plain layouts whose rows are whole 32-k groups of aligned bytes; false when
-// it does not apply (the kernel's offsets are 32 bits from a tile's first row) or the k-split
-// kernel, if it does (`ksplit`), is the faster one.
 template <int OUT>
-bool launch_w4a8_tile(const W4A8Args &a, bool ksplit, hipStream_t s)
+void launch_w4a8_tile(const W4A8Args &a, W4A8Route route, hipStream_t s)
 {
-    if (!tile_layout(a)) {
-        return false;
-    }
     TileArgs t = tile_args(a);
     constexpr int kElem = OUT == OUT_F32 ? 4 : 2;
     t.vec_d = a.ldd % 4 == 0 && reinterpret_cast<uintptr_t>(a.D) % (4 * kElem) == 0;
-    int best = 0;
-    const float best_us = w4a8_tile_us(a, best);
-    if (best_us == 0.f) {
-        return false;
-    }
-    const int passes = (a.M + kRowsPerChunk - 1) / kRowsPerChunk;
-    if (ksplit && 3.2f + 0.115e-6f * static_cast<float>(a.N) * static_cast<float>(a.K) *
-                              static_cast<float>(passes) <= best_us) {
-        return false;
-    }
-    switch (best) {
-    case 0: launch_tile<4, 2, 2, 4, 1, 3, OUT>(t, s); break;
-    case 1: launch_tile<4, 2, 1, 2, 2, 3, OUT>(t, s); break;
-    case 2: launch_tile<2, 2, 1, 2, 2, 4, OUT>(t, s); break;
+    switch (route) {
+    case W4A8_TILE_256X256: launch_tile<4, 2, 2, 4, 1, 3, OUT>(t, s); break;
+    case W4A8_TILE_128X128: launch_tile<4, 2, 1, 2, 2, 3, OUT>(t, s); break;
+    case W4A8_TILE_64X128: launch_tile<2, 2, 1, 2, 2, 4, OUT>(t, s); break;
     default: launch_tile<1, 2, 1, 2, 2, 6, OUT>(t, s); break;
     }
-    return true;
 }
 
 // Generic path: one thread per output, any alignment, any even k.
@@ -1014,12 +926,13 @@ void w4a8_run(size_t m, size_t n, size_t k, const void *A, size_t lda, size_t k_
                       aligned16(B) && (m + kRowsPerChunk - 1) / kRowsPerChunk < 65536 &&
                       lda < (1u << 24) && ldb / 2 < (1u << 24) && ldc < (1u << 24) &&
                       ldd < (1u << 24);
+    const W4A8Route route = packed || !tile_layout(a) ? W4A8_OTHER : w4a8_route(m, n, k, fast);
     if (fast && !packed && launch_w4a8_strip<OUT>(a, s)) {
         // decode strip kernel (m = 1, k = 2048 or 4096)
-    } else if (!packed && launch_w4a8_skinny<OUT>(a, fast, s)) {
-        // few-row kernel
-    } else if (!packed && launch_w4a8_tile<OUT>(a, fast, s)) {
-        // large-tile kernel
+    } else if (route == W4A8_FEW_ROW) {
+        launch_w4a8_skinny<OUT>(a, s);
+    } else if (route != W4A8_OTHER) {
+        launch_w4a8_tile<OUT>(a, route, s);
     } else if (fast) {
         const unsigned gx = static_cast<unsigned>((n + kNTile - 1) / kNTile);
         const unsigned long long gy = (m + kRowsPerChunk - 1) / kRowsPerChunk;

@@ -15,6 +15,147 @@ constexpr bool grid_fits(long long blocks, int threads)
     return blocks * threads < 0x100000000ll;
 }
 
+constexpr long long ceil_div(long long a, long long b)
+{
+    return (a + b - 1) / b;
+}
+
+// ---------------------------------------------------------------------------------------------
+// W4A8: the few-row kernel (int4_skinny.hpp), the tiles of int8_tile.hpp, or neither - the k-split
+// kernel where it applies (k a multiple of 256) and one thread per output otherwise.
+// ---------------------------------------------------------------------------------------------
+
+enum W4A8Route
+{
+    W4A8_OTHER,
+    W4A8_FEW_ROW,
+    W4A8_TILE_256X256,
+    W4A8_TILE_128X128,
+    W4A8_TILE_64X128,
+    W4A8_TILE_32X128
+};
+
+// Every tile is one pass of a CU over k, so a launch costs ceil(tiles / 256) times (fixed + stages *
+// rate) of its tile; the rates are microseconds measured on MI355X at k 864 and 4096 (M x N tiles:
+// 256 x 256 82 us for one round of 256 at k 4096, 128 x 128 23, 64 x 128 14.7, 32 x 128 11.7), and the
+// cheapest wins: 1000 x 11008 x 4096 takes 128 x 128 tiles (69 us; 74 with 256 x 256, 79 with 64 x
+// 128, 108 with 32 x 128), 512 x 4096 x 4096 64 x 128 (18.3; 25.7, 21.6 with 32 x 128), 4096^3 256 x
+// 256 (82; 97).
+struct W4A8Tile
+{
+    W4A8Route route;
+    int bm, bn, threads;
+    float fixed, stage;  // us per round: fixed + stage * ceil(k / 128)
+};
+constexpr W4A8Tile kW4A8Tiles[] = {{W4A8_TILE_256X256, 256, 256, 512, 18.0f, 2.0f},
+                                   {W4A8_TILE_128X128, 128, 128, 256, 5.0f, 0.57f},
+                                   {W4A8_TILE_64X128, 64, 128, 256, 4.5f, 0.32f},
+                                   {W4A8_TILE_32X128, 32, 128, 256, 4.0f, 0.24f}};
+
+// Microseconds of the cheapest tile, and which it is; 0 where no tile's grid fits.
+inline float w4a8_tile_us(long long M, long long N, long long K, W4A8Route &best)
+{
+    const float stages = static_cast<float>(ceil_div(K, 128));
+    float best_us = 0.f;
+    for (const W4A8Tile &p : kW4A8Tiles) {
+        const long long tiles = ceil_div(M, p.bm) * ceil_div(N, p.bn);
+        if (!grid_fits(tiles + 8, p.threads)) {
+            continue;
+        }
+        const float us = static_cast<float>(ceil_div(tiles, kTileCUs)) * (p.fixed + p.stage * stages);
+        if (best_us == 0.f || us < best_us) {
+            best = p.route;
+            best_us = us;
+        }
+    }
+    return best_us;
+}
+
+// Whether the few-row kernel is faster than the k-split kernel (k a multiple of 256, up to 32 rows).
+// Both give 16 channels (a strip) to a workgroup of eight waves that split k. The k-split kernel
+// requests all of a wave's weights at once, one pass per 15 rows, and stages up to 15 rows of all of
+// k in LDS; the few-row kernel keeps one or two blocks of 256 k in flight per wave and reads the
+// weights once for 32 rows. Measured on MI355X with each layer's weights from HBM, 110 shapes of 4 to
+// 1813 strips and k 256 to 16128 (few-row, k-split, us):
+//   up to 8 rows
+//     k to 1024: few-row (2 x 16384 x 512 3.8, 4.5; 4 x 1024 x 1024 2.5, 2.6)
+//     k to 2048: few-row, but k-split to four rows and two strips a CU (2 x 2048 x 2048 3.4, 3.1; 2 x
+//       18720 x 1792 1.12 times faster in few rows)
+//     k to 4096: k-split, whose one or two loads a wave are all in flight (8 x 4096 x 4096 4.6, 4.3; 2 x
+//       11008 x 4096 6.4, 6.1; 2 x 6272 x 2816 5.2, 4.4), but few-row over three strips a CU to k 3072
+//       (8 x 15712 x 3072 7.5, 8.2)
+//     longer k, strips that leave CUs idle: few-row (2 x 896 x 13824 5.5, 6.6; 8 rows 5.9, 8.8), but
+//       k-split for one row to k 8192 (1 x 272 x 4608 3.5, 3.3)
+//     longer k, more strips: the k-split kernel while two of its workgroups share a CU (1 x 8192 x 8192
+//       9.8, 7.8; 8 rows 9.9, 9.1; 2 x 5120 x 13824 11.2, 10.0), the few-row kernel where its staged
+//       rows no longer let them (8 x 5120 x 13824 12.9, 15.3; 8 x 17648 x 9472 1.4 times faster; 4 x
+//       9008 x 11264 12.5, 14.0) or it runs over two strips a CU with five rows and more (8 x 12080 x
+//       4608 1.2 times)
+//   9 to 16 rows: few-row (12 x 6352 x 4608 7.1, 8.5), but 9 x 8192 x 8192 11.3, 10.2
+//   17 to 32 rows, where the k-split kernel makes two or three passes: few-row (32 x 11008 x 4096 13.1,
+//     19.2), but k-split where its passes fit a workgroup a CU (17 x 1280 x 3840 4.7, 4.2) and for
+//     short k (24 x 2048 x 2048 4.2, 3.6; 17 x 16384 x 512 8.9, 7.2), three passes over more than a
+//     strip a CU aside (32 x 7616 x 1280 5.9, 7.4)
+inline bool w4a8_few_row_beats_ksplit(long long M, long long N, long long K)
+{
+    const long long strips = ceil_div(N, 16);
+    if (M <= 8) {
+        if (K <= 2048) {
+            return K <= 1024 || M > 4 || strips > 2 * kTileCUs;
+        }
+        if (K <= 4096) {
+            return K <= 3072 && strips > 3 * kTileCUs;
+        }
+        if (strips <= 224) {
+            return M > 1 || K > 8192;
+        }
+        if (K > 8192) {
+            return strips <= 256 || M >= 5 || (M == 4 && strips > 512);
+        }
+        return M >= 5 && strips > 512;
+    }
+    if (M <= 16) {
+        return !(M <= 10 && K > 6144 && K <= 8192 && strips > 224 && strips <= 512);
+    }
+    const long long passes = ceil_div(M, 15);
+    if (K > 4096) {
+        return true;
+    }
+    if (K > 2048) {
+        return strips * passes > 256;
+    }
+    return passes == 3 && K >= 1024 && strips > 224 && strips <= 512;
+}
+
+// Plain operands in the tile kernels' layout. ksplit: the k-split kernel applies (else one thread per
+// output is the alternative, which both others always beat).
+// The few-row kernel against the tiles, past 8 rows: the activations weigh as much as the weights and
+// each strip reloads them (16 x 28672 x 8192 26.7 us, 24 in tiles; 32 x 28672 x 8192 35, 24).
+// The k-split kernel against the tiles: one pass over the weights per 15 rows, 3.2 us + 0.115 us per
+// 10^6 weights and pass (11008 x 4096: 12.6 us at 16 rows, 18.5 at 32, 23.0 at 48, against 12.2-12.8
+// in tiles; 4096 x 4096: 9.7 at 48 and 27.1 at 200, against 12.5 and 12.8).
+inline W4A8Route w4a8_route(long long M, long long N, long long K, bool ksplit)
+{
+    W4A8Route tile = W4A8_OTHER;
+    const float tile_us = w4a8_tile_us(M, N, K, tile);
+    const long long strips = ceil_div(N, 16);
+    if (M <= 32 && grid_fits(strips, 512) && (!ksplit || w4a8_few_row_beats_ksplit(M, N, K))) {
+        const float rate = (M > 16 ? 2.3f : 1.5f) / 4096.f;
+        const float us = 3.4f + rate * static_cast<float>(ceil_div(strips, kTileCUs)) *
+                                    static_cast<float>(K);
+        if (M <= 8 || us <= tile_us) {
+            return W4A8_FEW_ROW;
+        }
+    }
+    // (up to 8 rows a pass costs the k-split kernel 0.08 us per 10^6 weights: never in tiles)
+    if (tile_us == 0.f || (ksplit && M <= 8) ||
+        (ksplit && 3.2f + 0.115e-6f * static_cast<float>(N) * static_cast<float>(K) *
+                              static_cast<float>(ceil_div(M, 15)) <= tile_us)) {
+        return W4A8_OTHER;
+    }
+    return tile;
+}
+
 // ---------------------------------------------------------------------------------------------
 // W4A16
 // ---------------------------------------------------------------------------------------------
