@@ -14,6 +14,7 @@ def rules(route):
     route.tqtr_first_wrong_scale_block.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
     route.tqtr_w4a16_skinny_scales_exact.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
     route.tqtr_w4a8_route.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
+    route.tqtr_w8a8_few_row.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
     return route
 
 
@@ -65,3 +66,19 @@ def test_w4a8_few_rows(rules, m, n, k, ksplit):
     assert rules.tqtr_w4a8_route(m, n, k, 1) == want
     # off the 256 grid of k the few-row kernel has only the tiles beside it
     assert rules.tqtr_w4a8_route(m, n, k + 32, 0) != T.W4A8_OTHER
+
+
+# (m, n, k, dynamic, packed, whether the few-row kernel was the faster one), measured side by side with
+# the weights from HBM, where the two differ by 8% and more
+@pytest.mark.parametrize("m,n,k,dyn,packed,few", [
+    (1, 4096, 4096, 0, 0, True), (32, 4096, 4096, 0, 0, True), (8, 4096, 4096, 1, 0, True),
+    (1, 28672, 8192, 0, 0, True), (8, 28672, 8192, 1, 0, True), (16, 4096, 11008, 0, 1, True),
+    (32, 11008, 4096, 0, 0, True), (17, 16384, 4096, 1, 0, True), (33, 4096, 4096, 0, 0, True),
+    (64, 512, 2048, 1, 0, True), (16, 1024, 4112, 0, 0, True),
+    (1, 16384, 512, 0, 0, False), (16, 16384, 512, 0, 0, False), (9, 16384, 512, 1, 0, False),
+    (17, 16384, 4096, 0, 0, False), (24, 28672, 8192, 0, 0, False), (32, 28672, 8192, 0, 1, False),
+    (1, 23232, 128, 0, 0, False), (16, 23232, 128, 1, 0, False), (32, 26768, 384, 0, 1, False),
+    (65, 23232, 128, 0, 0, False), (65, 23232, 128, 1, 0, False), (64, 11008, 4096, 0, 0, False),
+])
+def test_w8a8_few_rows(rules, m, n, k, dyn, packed, few):
+    assert rules.tqtr_w8a8_few_row(m, n, k, dyn, packed) == few

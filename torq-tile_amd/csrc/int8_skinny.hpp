@@ -240,31 +240,18 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void int8_skinny_kernel(Int8Args
     }
 }
 
-// The few-row kernel where it is the faster one and the strides fit its 32-bit offsets. Measured on
-// MI355X (f16 results, us, per-row quantized; the stream kernel in parentheses): 4096 x 4096 at 8
-// rows 6.4 (17.1), 32 rows 7.1 (19.3), 64 rows 11.5 (19.5); 11008 x 4096 at 8 rows 11.8 (18.4), 32
-// rows 15.9 (21.5), 64 rows 32 (22.8); 4096 x 11008 at 8 rows 13.1 (38.8), 64 rows 24 (47). Up to
-// 32 rows it always wins; past them every 32 rows are a pass over the weights, about 4 us + 0.29 us
-// per 10^6 weights and pass, against 3 us + 0.5 us per 128 of k for each round of the stream
-// kernel's 64-row tiles.
+// The few-row kernel where it is the faster one (route.hpp) and the strides fit its 32-bit offsets.
 // Ring depth: 2 blocks (1 from 17 rows on) measured as fast as 3 or 4 at 4096 channels and faster at
 // 11008 (11.8 against 12.4 and 15.8 us at 8 rows), where the smaller ring lets two or three
 // workgroups share a CU.
 template <int EPI, int PK>
 bool launch_skinny(const Int8Args &a, hipStream_t stream)
 {
-    const int passes = (a.M + 31) / 32;
-    if (!grid_fits((a.N + kSkinnyN - 1) / kSkinnyN, 64 * kSkinnyWaves) || passes > 4 || a.K == 0 || a.lda >= (1 << 22) || a.ldb >= (1 << 22)) {
+    if (a.lda >= (1 << 22) || a.ldb >= (1 << 22) ||
+        !w8a8_few_row(a.M, a.N, a.K, is_dyn(EPI), PK != PK_NONE)) {
         return false;
     }
-    if (passes > 1) {
-        const float mw = 1e-6f * static_cast<float>(a.N) * static_cast<float>(a.K);
-        const int rounds = (((a.M + 63) / 64) * ((a.N + kBN - 1) / kBN) + 255) / 256;
-        if (4.0f + 0.29f * mw * static_cast<float>(passes) >
-            static_cast<float>(rounds) * (3.0f + 0.5f * static_cast<float>(a.K) / 128.0f)) {
-            return false;
-        }
-    }
+    const int passes = (a.M + 31) / 32;
     const unsigned gx = static_cast<unsigned>((a.N + kSkinnyN - 1) / kSkinnyN);
     const dim3 block(kSkinnyWaves * 64);
     if (a.M <= 8) {

@@ -157,6 +157,57 @@ inline W4A8Route w4a8_route(long long M, long long N, long long K, bool ksplit)
 }
 
 // ---------------------------------------------------------------------------------------------
+// W8A8 with B = [n, k], static and per-row quantized ("dynamic") activations, plain or packed operands.
+// ---------------------------------------------------------------------------------------------
+
+// Whether the few-row kernel (int8_skinny.hpp; 16 channels and 32 rows a workgroup) is faster than what
+// takes the shape otherwise: the stream kernel (k a multiple of 128), or the double-buffered one. Both
+// sides in microseconds, fitted on MI355X with each layer's weights from HBM over 45 shapes of 128 to
+// 2048 strips of 16 channels, k 64 to 14336, and 9 row counts to 32 (the pick is within 6% of the
+// better one but for a few points, at most 18%; always the few-row kernel was up to 97% slower):
+//   few-row: a workgroup's fixed part and its share of k, by rounds of 256 of them, more with the
+//     activation rows that every strip loads too (f32 results: 8 x 4096 x 4096 6.4 us, 16.8 in the
+//     stream kernel; static: 1 x 11008 x 4096 11.6, 15.6; 32 x 11008 x 4096 15.9, 17.5)
+//   stream kernel: a serial walk over k of 128-channel tiles, then their number and the bytes of the
+//     weights (static: 9 x 16384 x 512 5.0, few-row 6.7; 16 x 23232 x 128 4.6, 8.4; 32 x 28672 x 8192 51, 63)
+// Past 32 rows every 32 rows are a pass over the weights, about 4 us + 0.29 us per 10^6 weights and
+// pass and no less than a workgroup's fixed part, against 3 us + 0.5 us per 128 of k for each round of
+// the stream kernel's 64-row tiles (64 x 4096 x 4096 11.5 us, 19.5; 65 x 23232 x 128 20.6, 5.8).
+inline bool w8a8_few_row(long long M, long long N, long long K, bool dyn, bool packed)
+{
+    const long long strips = ceil_div(N, 16);
+    const long long passes = ceil_div(M, 32);
+    if (passes > 4 || K <= 0 || !grid_fits(strips, 512)) {
+        return false;
+    }
+    const float rounds = strips < kTileCUs ? 1.f : static_cast<float>(strips) / kTileCUs;
+    const float mw = 1e-6f * static_cast<float>(N) * static_cast<float>(K);
+    if (passes > 1) {
+        const float by_bytes = 4.0f + 0.29f * mw * static_cast<float>(passes);
+        const float by_count = 2.2f + rounds * static_cast<float>(passes);
+        const float stream = static_cast<float>(ceil_div(ceil_div(M, 64) * ceil_div(N, 128), kTileCUs)) *
+                             (3.0f + 0.5f * static_cast<float>(K) / 128.0f);
+        return (by_bytes > by_count ? by_bytes : by_count) <= stream;
+    }
+    const float rows = static_cast<float>(M);
+    const float fixed = (M <= 8 ? 0.66f : 1.0f) + (dyn ? 0.2f : 0.f);
+    const float rate = (M <= 8 ? 2.55f : (M <= 16 ? 2.95f : 3.6f)) * (packed ? 1.05f : 1.f);
+    const float few = 2.2f + rounds * (fixed + rate * static_cast<float>(K) / 4096.f);
+    const float tiles = static_cast<float>(ceil_div(N, 128)) / kTileCUs;
+    const float stages = static_cast<float>(ceil_div(K, 128));
+    float other;
+    if (K % 128 == 0) {
+        other = dyn ? 2.95f + 0.36f * stages + 2.6f * tiles + 0.067f * mw + 0.075f * rows
+                    : 2.9f + 0.28f * stages + 1.5f * tiles + 0.078f * mw + 0.02f * rows;
+    } else {
+        other = dyn ? 3.9f + 0.8f * stages + 2.6f * tiles + 0.0124f * mw + 0.14f * rows
+                    : 4.1f + (packed ? 0.6f : 0.75f) * stages + 1.6f * tiles + 0.025f * mw + 0.12f * rows;
+    }
+    const float by_bytes = 2.f + mw / (dyn ? 4.3f : 4.9f);
+    return few < (other > by_bytes ? other : by_bytes);
+}
+
+// ---------------------------------------------------------------------------------------------
 // W4A16
 // ---------------------------------------------------------------------------------------------
 
