@@ -20,6 +20,11 @@ int tqtr_w8a8_few_row(long long m, long long n, long long k, int dyn, int packed
     return w8a8_few_row(m, n, k, dyn != 0, packed != 0);
 }
 
+int tqtr_w8a8_tile(long long m, long long n, long long k, int dyn)
+{
+    return w8a8_tile(m, n, k, dyn != 0);
+}
+
 uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
 {
     return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));

@@ -15,6 +15,7 @@ def rules(route):
     route.tqtr_w4a16_skinny_scales_exact.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
     route.tqtr_w4a8_route.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     route.tqtr_w8a8_few_row.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
+    route.tqtr_w8a8_tile.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     return route
 
 
@@ -82,3 +83,16 @@ def test_w4a8_few_rows(rules, m, n, k, ksplit):
 ])
 def test_w8a8_few_rows(rules, m, n, k, dyn, packed, few):
     assert rules.tqtr_w8a8_few_row(m, n, k, dyn, packed) == few
+
+
+# (m, n, k, dynamic, whether large tiles were the faster ones), measured side by side
+@pytest.mark.parametrize("m,n,k,dyn,tiles", [
+    (4000, 11008, 4096, 0, True), (2048, 4096, 11008, 0, True), (2000, 4096, 4096, 1, True),
+    (1000, 4096, 4112, 0, True), (313, 13616, 1280, 0, True), (2048, 4096, 512, 1, True),
+    (998, 6880, 192, 0, True), (2572, 1968, 352, 0, True),
+    (2048, 4096, 1024, 0, False), (2048, 4096, 512, 0, False), (551, 30304, 128, 0, False),
+    (133, 22176, 256, 0, False), (1000, 4096, 4096, 0, False), (512, 4096, 4112, 0, False),
+    (64, 32544, 3104, 0, False),
+])
+def test_w8a8_large_tiles(rules, m, n, k, dyn, tiles):
+    assert (rules.tqtr_w8a8_tile(m, n, k, dyn) != T.W8A8_NO_TILE) == tiles

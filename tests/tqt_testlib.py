@@ -16,9 +16,11 @@ ORACLE_SO = os.path.join(ROOT, "oracle", "liboracle.so")
 REF_SO = os.path.join(ROOT, "oracle", "_ref", "libtqt_ref.so")
 SHIM_SO = os.path.join(ROOT, "tests", "abi_shim", "libtqt_test_shim.so")
 ROUTE_SO = os.path.join(ROOT, "tests", "abi_shim", "libtqt_route_shim.so")
-# the W4A8Route values of torq-tile_amd/csrc/route.hpp
+# torq-tile_amd/csrc/route.hpp: W4A8Route
 (W4A8_OTHER, W4A8_FEW_ROW, W4A8_TILE_256X256, W4A8_TILE_128X128, W4A8_TILE_64X128,
  W4A8_TILE_32X128) = range(6)
+# W8A8Tile
+W8A8_NO_TILE, W8A8_TILE_128X128, W8A8_TILE_256X256 = range(3)
 GOLDEN_DIR = os.path.join(ROOT, "tests", "golden")
 
 c_size = ctypes.c_size_t

@@ -207,6 +207,54 @@ inline bool w8a8_few_row(long long M, long long N, long long K, bool dyn, bool p
     return few < (other > by_bytes ? other : by_bytes);
 }
 
+// Which large tile (w8a8_tile.hpp) takes a shape, if any. Rounds of 256 tiles, one per CU (the 128 x 128
+// tiles also two: a pair of rounds), in microseconds of fixed + rate * ceil(k / 128), measured on MI355X
+// at k 512, 4096 and 11008 with requantized (per-row dynamic, f32) results:
+//   stream kernel 128 x 128   3 + 0.67 n (3 + 1.0 n)
+//   128 x 128                 4 + 0.7 n (6 + 0.9 n), a pair 5 + 1.2 n (6 + 1.5 n)
+//   256 x 256                 14 + 1.5 n (20 + 1.8 n); the MFMAs alone are 1.37 n at the clock the
+//                             chip holds under them, the fixed part is the launch, the first loads
+//                             and 6 us of requantization that nothing overlaps
+// 4000 x 11008 x 4096 runs 256 x 256 tiles in 179 us (218 with 128 x 128, 255 on the stream kernel),
+// 2048 x 4096 x 11008 128 x 128 tiles in 95 (114), 2000 x 4096 x 4096 dynamic f32 in 53 (66); one
+// round, as 1000 x 4096 x 4096, stays on the stream kernel (24.5 us, 27 with 128 x 128 tiles).
+// Requantized results of a short k stay there too: the epilogue is most of such a launch, and the
+// stream kernel's overlaps better (2048 x 4096 x 1024 15.1 us, 15.8 in tiles; 551 x 30304 x 128 16.9,
+// 20.2; 1201 x 15968 x 128 17.7, 20.0; from k 1280 the tiles win, 313 x 13616 x 1280 14.9, 16.5).
+// k not a multiple of 128 has the double-buffered kernel instead of the stream kernel, which one nearly
+// full round of large tiles beats too (1000 x 4096 x 4112: 32.1 us, 41.2 there) and a half full one does
+// not (512 x 4096 x 4112: 30 us, 27 there), nor tiles half of whose rows are past the last (64 x 32544
+// x 3104: 27.9 us, 24.0 there, on 64-row tiles).
+enum W8A8Tile
+{
+    W8A8_NO_TILE,
+    W8A8_TILE_128X128,
+    W8A8_TILE_256X256
+};
+
+inline W8A8Tile w8a8_tile(long long M, long long N, long long K, bool dyn)
+{
+    const bool other = K % 128 != 0;
+    if (K <= 0 || (!dyn && !other && K <= 1024) || (other && M <= 64)) {
+        return W8A8_NO_TILE;
+    }
+    const float n = static_cast<float>(ceil_div(K, 128));
+    const long long t128 = ceil_div(M, 128) * ceil_div(N, 128);
+    const long long t256 = ceil_div(M, 256) * ceil_div(N, 256);
+    const long long r128 = ceil_div(t128, kTileCUs);
+    const float stream_us = static_cast<float>(r128) *
+                            (other ? 3.f + 1.2f * n : (dyn ? 3.f + 1.0f * n : 3.f + 0.67f * n));
+    const float mid_us = static_cast<float>(r128 / 2) * (dyn ? 6.f + 1.5f * n : 5.f + 1.2f * n) +
+                         static_cast<float>(r128 % 2) * (dyn ? 6.f + 0.9f * n : 4.f + 0.7f * n);
+    const float big_us =
+        static_cast<float>(ceil_div(t256, kTileCUs)) * (dyn ? 20.f + 1.8f * n : 14.f + 1.5f * n);
+    if (!grid_fits(t256 + 8, 512) || !grid_fits(t128 + 8, 256) ||
+        t128 <= (other ? 3 * kTileCUs / 4 : kTileCUs) || (stream_us <= mid_us && stream_us <= big_us)) {
+        return W8A8_NO_TILE;
+    }
+    return big_us < mid_us ? W8A8_TILE_256X256 : W8A8_TILE_128X128;
+}
+
 // ---------------------------------------------------------------------------------------------
 // W4A16
 // ---------------------------------------------------------------------------------------------

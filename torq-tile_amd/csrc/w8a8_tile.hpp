@@ -419,49 +419,19 @@ void launch_w8_tile(const Int8Args &a, hipStream_t stream)
                        stream, a, tiles_m, tiles_n, per_xcd, vec_d);
 }
 
-// The large tiles where they are faster than the stream kernel and the strides fit their 32-bit
-// offsets. Rounds of 256 tiles, one per CU (the 128 x 128 tiles also two: a pair of rounds), in
-// microseconds of fixed + rate * ceil(k / 128), measured on MI355X at k 512, 4096 and 11008 with
-// requantized (per-row dynamic, f32) results:
-//   stream kernel 128 x 128   3 + 0.67 n (3 + 1.0 n)
-//   128 x 128                 4 + 0.7 n (6 + 0.9 n), a pair 5 + 1.2 n (6 + 1.5 n)
-//   256 x 256                 14 + 1.5 n (20 + 1.8 n); the MFMAs alone are 1.37 n at the clock the
-//                             chip holds under them, the fixed part is the launch, the first loads
-//                             and 6 us of requantization that nothing overlaps
-// 4000 x 11008 x 4096 runs 256 x 256 tiles in 185 us (218 with 128 x 128, 261 on the stream kernel),
-// 2048 x 4096 x 11008 128 x 128 tiles in 106 (118), 2000 x 4096 x 4096 dynamic f32 in 54 (69); one
-// round, as 1000 x 4096 x 4096, stays on the stream kernel (24.5 us, 27 with 128 x 128 tiles).
+// The large tiles where they are the faster ones (route.hpp) and the strides fit their 32-bit offsets.
 template <int EPI, int PK>
 bool launch_w8a8_tile(const Int8Args &a, hipStream_t stream)
 {
-    if (a.K == 0 || a.lda >= (1 << 22) || a.ldb >= (1 << 22)) {
+    if (a.lda >= (1 << 22) || a.ldb >= (1 << 22)) {
         return false;
     }
     constexpr bool kDyn = is_dyn(EPI);
-    const float n = static_cast<float>((a.K + kTileK - 1) / kTileK);
-    auto rounds = [&](int b) {
-        return (static_cast<long long>((a.M + b - 1) / b) * ((a.N + b - 1) / b) + kTileCUs - 1) /
-               kTileCUs;
-    };
-    const long long r128 = rounds(128), r256 = rounds(256);
-    const float fr = static_cast<float>(r128);
-    // k not a multiple of 128 has the double-buffered kernel instead of the stream kernel, which one
-    // nearly full round of large tiles beats too (1000 x 4096 x 4112: 32.5 us, 41 there) and a half
-    // full one does not (512 x 4096 x 4112: 30 us, 27 there)
-    const bool other = a.K % kTileK != 0;
-    const float stream_us =
-        fr * (other ? 3.f + 1.2f * n : (kDyn ? 3.f + 1.0f * n : 3.f + 0.67f * n));
-    const float mid_us =
-        static_cast<float>(r128 / 2) * (kDyn ? 6.f + 1.5f * n : 5.f + 1.2f * n) +
-        static_cast<float>(r128 % 2) * (kDyn ? 6.f + 0.9f * n : 4.f + 0.7f * n);
-    const long long t256 = static_cast<long long>((a.M + 255) / 256) * ((a.N + 255) / 256);
-    const float big_us = static_cast<float>(r256) * (kDyn ? 20.f + 1.8f * n : 14.f + 1.5f * n);
-    const long long t128 = static_cast<long long>((a.M + 127) / 128) * ((a.N + 127) / 128);
-    if (!grid_fits(t256 + 8, 512) || !grid_fits(t128 + 8, 256) ||
-        t128 <= (other ? 3 * kTileCUs / 4 : kTileCUs) || (stream_us <= mid_us && stream_us <= big_us)) {
+    const W8A8Tile tile = w8a8_tile(a.M, a.N, a.K, kDyn);
+    if (tile == W8A8_NO_TILE) {
         return false;
     }
-    if (big_us < mid_us) {
+    if (tile == W8A8_TILE_256X256) {
         launch_w8_tile<4, 2, 2, 4, 1, 2, EPI, PK>(a, stream);
     } else if constexpr (kDyn) {
         // two k groups: 128 x 64 per wave, the channel sums' dot products over half the k-steps
