@@ -25,6 +25,11 @@ int tqtr_w8a8_tile(long long m, long long n, long long k, int dyn)
     return w8a8_tile(m, n, k, dyn != 0);
 }
 
+int tqtr_int8_edge_faster(int form, long long m, long long n, long long k, long long taps)
+{
+    return int8_edge_faster(static_cast<EdgeForm>(form), m, n, k, taps);
+}
+
 uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
 {
     return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));

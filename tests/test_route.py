@@ -16,6 +16,7 @@ def rules(route):
     route.tqtr_w4a8_route.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     route.tqtr_w8a8_few_row.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
     route.tqtr_w8a8_tile.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
+    route.tqtr_int8_edge_faster.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
     return route
 
 
@@ -96,3 +97,22 @@ def test_w8a8_few_rows(rules, m, n, k, dyn, packed, few):
 ])
 def test_w8a8_large_tiles(rules, m, n, k, dyn, tiles):
     assert (rules.tqtr_w8a8_tile(m, n, k, dyn) != T.W8A8_NO_TILE) == tiles
+
+
+# (form, m, n, k, taps, whether the 64 x 64 tiles were the faster ones), measured side by side, 15% apart
+# and more
+@pytest.mark.parametrize("form,m,n,k,taps,tiles", [
+    (T.EDGE_NK, 64, 64, 44, 0, False), (T.EDGE_NK, 17, 33, 40, 0, False),
+    (T.EDGE_NK, 200, 255, 41, 0, False), (T.EDGE_NK, 32, 256, 40, 0, False),
+    (T.EDGE_NK, 1, 16, 36, 0, False), (T.EDGE_NK, 1, 255, 100, 0, True),
+    (T.EDGE_NK, 200, 4097, 33, 0, True), (T.EDGE_NK, 64, 255, 130, 0, True),
+    (T.EDGE_KN_CLAMP, 200, 255, 33, 0, False), (T.EDGE_KN_CLAMP, 17, 33, 40, 0, False),
+    (T.EDGE_KN_CLAMP, 1, 255, 65, 0, True), (T.EDGE_KN_CLAMP, 64, 1023, 100, 0, True),
+    (T.EDGE_KN_CLAMP, 512, 4097, 33, 0, True),
+    (T.EDGE_KN_REQUANT, 64, 255, 81, 0, False), (T.EDGE_KN_REQUANT, 16, 1023, 100, 0, True),
+    (T.EDGE_CONV, 784, 32, 27, 9, False), (T.EDGE_CONV, 12544, 8, 27, 9, False),
+    (T.EDGE_CONV, 12544, 32, 24, 1, False), (T.EDGE_CONV, 12544, 96, 27, 9, True),
+    (T.EDGE_CONV, 784, 32, 147, 49, True), (T.EDGE_CONV, 49, 32, 49, 49, True),
+])
+def test_int8_edge(rules, form, m, n, k, taps, tiles):
+    assert rules.tqtr_int8_edge_faster(form, m, n, k, taps) == tiles

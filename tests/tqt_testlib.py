@@ -19,6 +19,8 @@ ROUTE_SO = os.path.join(ROOT, "tests", "abi_shim", "libtqt_route_shim.so")
 # torq-tile_amd/csrc/route.hpp: W4A8Route
 (W4A8_OTHER, W4A8_FEW_ROW, W4A8_TILE_256X256, W4A8_TILE_128X128, W4A8_TILE_64X128,
  W4A8_TILE_32X128) = range(6)
+# EdgeForm
+EDGE_NK, EDGE_KN_CLAMP, EDGE_KN_REQUANT, EDGE_CONV = range(4)
 # W8A8Tile
 W8A8_NO_TILE, W8A8_TILE_128X128, W8A8_TILE_256X256 = range(3)
 GOLDEN_DIR = os.path.join(ROOT, "tests", "golden")

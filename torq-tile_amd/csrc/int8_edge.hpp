@@ -248,14 +248,16 @@ __global__ __launch_bounds__(256) void int8_edge_kernel(Int8Args a)
     }
 }
 
-// All but a few outputs of a short k, which one thread each finishes before a stage is staged (us, one
-// thread per output in parentheses: 4 x 4 x 20 4.7 (3.2), 17 x 33 x 100 5.8 (8.9), 1 x 4097 x 4000 49
-// (413); convolutions, whose fetch is dearer: 14 x 14 x 24 to 32 channels, 1 x 1, 11.8 (5.3), 28 x 28
-// x 3 to 32, 3 x 3, 12.9 (7.4), 4 x 112 x 112 x 3 to 64, 7 x 7, 17 (130)).
 template <int AM, int BMd, int EPI>
 bool launch_edge(const Int8Args &a, hipStream_t stream)
 {
-    if (a.K <= (AM == A_CONV_CL ? 48 : 32) && static_cast<long long>(a.M) * a.N <= 32768) {
+    constexpr EdgeForm form = AM == A_CONV_CL       ? EDGE_CONV
+                              : BMd == B_NK         ? EDGE_NK
+                              : EPI == EPI_CLAMP_I32 ? EDGE_KN_CLAMP
+                                                     : EDGE_KN_REQUANT;
+    const long long taps = AM == A_CONV_CL
+                               ? static_cast<long long>(a.cv.KD) * a.cv.KH * a.cv.KW : 0;
+    if (!int8_edge_faster(form, a.M, a.N, a.K, taps)) {
         return false;
     }
     const long long blocks = static_cast<long long>((a.M + kEdgeT - 1) / kEdgeT) *

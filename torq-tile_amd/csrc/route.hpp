@@ -256,6 +256,55 @@ inline W8A8Tile w8a8_tile(long long M, long long N, long long K, bool dyn)
 }
 
 // ---------------------------------------------------------------------------------------------
+// Int8 products and convolutions off the 16-byte grid: 64 x 64 MFMA tiles (int8_edge.hpp) or one thread
+// per output, which finishes a short k before a stage is staged.
+// ---------------------------------------------------------------------------------------------
+
+enum EdgeForm
+{
+    EDGE_NK,          // B = [n, k], requantized
+    EDGE_KN_CLAMP,    // B = [k, n], int32 results
+    EDGE_KN_REQUANT,  // B = [k, n], requantized
+    EDGE_CONV         // channel-last implicit convolution (M pixels, N channels)
+};
+
+// Whether the tiles are faster. Microseconds of both on MI355X, fitted over M 1 to 512, N 15 to 4097, k
+// 1 to 200 and 273 convolutions of 1 to 40 channels and 1 to 49 taps, the pick never over 26% from the
+// better one:
+//   a thread per output: a launch and k steps of one thread, more once the outputs fill the chip (64 x
+//     64 x 44 5.5 us, in tiles 9.9; 200 x 4097 x 33 requantized 31.9, in tiles 8.5)
+//   tiles: a launch, the epilogue of up to 64 rows and, for a k that ends inside a 16-byte load, its last
+//     bytes one by one (64 x 255 requantized: k 33 8.2, k 41 9.7); more where every row has a multiplier
+//     of its own (64 x 255 x 81 12.8, a thread per output 10.8); a convolution's taps byte by byte
+//     (28 x 28 x 3 to 32, 3 x 3, 12.9, a thread per output 7.5; 112 x 112 x 3 to 96 14.3, 31.8)
+inline bool int8_edge_faster(EdgeForm form, long long M, long long N, long long K, long long taps)
+{
+    const float outs = static_cast<float>(M) * static_cast<float>(N);
+    const float tiles = static_cast<float>(ceil_div(M, 64)) * static_cast<float>(ceil_div(N, 64));
+    const float k = static_cast<float>(K);
+    const float rows = M < 64 ? static_cast<float>(M) : 64.f;
+    const float tail = static_cast<float>(K % 16);
+    auto larger = [](float a, float b) { return a > b ? a : b; };
+    float thread_us, tile_us;
+    switch (form) {
+    case EDGE_NK:
+        thread_us = 2.7f + k * larger(0.066f, (K <= 32 ? 0.75e-6f : 1.15e-6f) * outs);
+        tile_us = 4.9f + 0.05f * rows + 0.16f * tail + 0.003f * tiles;
+        break;
+    case EDGE_CONV:
+        thread_us = 4.f + 0.065f * k + 0.2f * static_cast<float>(taps) +
+                    1e-6f * outs * (3.f + 0.5f * k + 0.5f * static_cast<float>(taps));
+        tile_us = 12.f + tiles * (0.009f + 0.00013f * k);
+        break;
+    default:
+        thread_us = 2.3f + k * larger(N < 64 ? 0.07f : 0.1f, 0.28e-6f * outs);
+        tile_us = (form == EDGE_KN_CLAMP ? 4.6f + 0.028f * rows : 4.9f + 0.105f * rows) + 0.02f * k +
+                  0.1f * tail + 0.003f * tiles;
+    }
+    return tile_us < thread_us;
+}
+
+// ---------------------------------------------------------------------------------------------
 // W4A16
 // ---------------------------------------------------------------------------------------------
 
