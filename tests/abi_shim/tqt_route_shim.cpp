@@ -30,6 +30,13 @@ int tqtr_int8_edge_faster(int form, long long m, long long n, long long k, long 
     return int8_edge_faster(static_cast<EdgeForm>(form), m, n, k, taps);
 }
 
+// the kernel, and in hundreds its blocks per compensation
+int tqtr_w4a16_route(long long m, long long n, long long k, long long bl, int f32, int other)
+{
+    const W4A16Route r = w4a16_route(m, n, k, bl, f32 != 0, static_cast<W4A16Other>(other));
+    return r.kernel + 100 * r.comp;
+}
+
 uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
 {
     return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));

@@ -121,3 +121,25 @@ def test_w4a16_tile_infinity(gpu, bl):
     rest = np.ones(m, bool)
     rest[[7, 9]] = False
     assert np.isfinite(got[rest]).all()
+
+
+@pytest.mark.parametrize("m,n,k,comp", [(256, 4096, 1024, 1), (256, 4096, 2048, 2),
+                                        (256, 4096, 4096, 4), (300, 2050, 8192, 8),
+                                        (1000, 1040, 640, 8)])
+def test_w4a16_tile_f16_sums(gpu, shim, route, m, n, k, comp):
+    """f16 results keep the sums of 32-wide blocks as exact as the chunk-stream and register kernels do
+    (relative error 4.8e-8 at k 1024 to 8.2e-8 at 8192; 9.6e-8 for the register kernel's). C cancels all
+    but the last bits of each sum, so that its error shows beside the 11 bits of the result: at most
+    1e-7 of the sums' rms here, where plain f32 accumulators are off by 1.06e-7 (k 1024), 1.5e-7 (2048),
+    2.0e-7 (4096) and 2.9e-7 (8192). The results' own rounding adds at most 2^-12 of a difference of at
+    most 2^-11 of the sum: 3.5e-8."""
+    route.tqtr_w4a16_route.argtypes = [ctypes.c_longlong] * 4 + [ctypes.c_int] * 2
+    got = route.tqtr_w4a16_route(m, n, k, 32, 0, T.W4A16_CHUNK if k % 512 == 0 else T.W4A16_REGISTER)
+    assert got % 100 >= T.W4A16_TILE_128X256 and got // 100 == comp
+    d = T.gen_w4a16(m, n, k, bl=32, seed=k, with_bias=False)
+    v, _ = _exact(d)
+    d["C16"] = T.f16_bits(-v)
+    out = T.bits_f16(_gr().run_w4a16(shim, d, 0xFBFF, 0x7BFF)).astype(np.float64)
+    left = v + T.bits_f16(d["C16"]).astype(np.float64)
+    err = np.sqrt(np.mean((out - left) ** 2) / np.mean(v ** 2))
+    assert err <= 1e-7, err

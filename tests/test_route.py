@@ -17,6 +17,7 @@ def rules(route):
     route.tqtr_w8a8_few_row.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
     route.tqtr_w8a8_tile.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     route.tqtr_int8_edge_faster.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
+    route.tqtr_w4a16_route.argtypes = [ctypes.c_longlong] * 4 + [ctypes.c_int] * 2
     return route
 
 
@@ -116,3 +117,17 @@ def test_w8a8_large_tiles(rules, m, n, k, dyn, tiles):
 ])
 def test_int8_edge(rules, form, m, n, k, taps, tiles):
     assert rules.tqtr_int8_edge_faster(form, m, n, k, taps) == tiles
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("k", [640, 1024, 2048, 4096, 11264])
+def test_w4a16_sums(rules, f32, k):
+    """32-wide blocks that another kernel sums in f64 or short chains are never left to plain f32
+    accumulators; blocks that only one thread per output takes otherwise may be."""
+    other = T.W4A16_CHUNK if k % 512 == 0 else T.W4A16_REGISTER
+    for m in (33, 64, 100, 256, 1024, 4000):
+        for n in (512, 4096, 14336):
+            r = rules.tqtr_w4a16_route(m, n, k, 32, f32, other)
+            assert r % 100 < T.W4A16_TILE_128X256 or r // 100 > 0
+    assert rules.tqtr_w4a16_route(1024, 4096, 11008, 128, f32, T.W4A16_GENERIC) == \
+        T.W4A16_TILE_128X128

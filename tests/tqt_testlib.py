@@ -19,6 +19,10 @@ ROUTE_SO = os.path.join(ROOT, "tests", "abi_shim", "libtqt_route_shim.so")
 # torq-tile_amd/csrc/route.hpp: W4A8Route
 (W4A8_OTHER, W4A8_FEW_ROW, W4A8_TILE_256X256, W4A8_TILE_128X128, W4A8_TILE_64X128,
  W4A8_TILE_32X128) = range(6)
+# W4A16Other, W4A16Kernel (the routes add 100 times the blocks per compensation)
+W4A16_GENERIC, W4A16_REGISTER, W4A16_CHUNK = range(3)
+(W4A16_OTHER, W4A16_FEW_ROW, W4A16_TILE_128X256, W4A16_TILE_128X128, W4A16_TILE_64X128,
+ W4A16_TILE_32X64) = range(6)
 # EdgeForm
 EDGE_NK, EDGE_KN_CLAMP, EDGE_KN_REQUANT, EDGE_CONV = range(4)
 # W8A8Tile

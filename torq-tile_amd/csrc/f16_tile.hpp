@@ -17,7 +17,9 @@
 //
 // Numerics: (q - 8) is exact in f16, products are exact in f32, one block's products are summed by
 // the MFMA in f32, and the block sum times the f32 value of its f16 scale is accumulated in f32
-// (one rounding) - the per-block scaling of the reference test's oracle.
+// (one rounding) - the per-block scaling of the reference test's oracle. With 32-wide blocks the
+// accumulators are compensated and meet in f64 wherever the kernel that the shape had before sums in
+// f64 or in shorter chains.
 //
 // LDS layout (conflict-free): activation row r's 16-byte chunk c at c ^ (r & 15) of its 256 bytes;
 // a weight row's 16 bytes of sub-step T at T ^ ((r >> 2) & 3) of its 64; scales as whole dwords (the
@@ -29,11 +31,10 @@
 // constant vmcnt. The barrier of a stage sits where its last fragments are in registers.
 //
 // Measured: 1024 x 4096 x 11008, 128-wide blocks, f32 results 114 us (318 ms on the per-output
-// kernel, the only one for blocks other than 32 wide); 32-wide blocks, f16 results, 128 x 4096 x
-// 4096 18.8 us (44.3 on the chunk-stream kernel, one pass over the weights per 32 rows) and 1024 x
-// 4096 x 4096 54 us (339); f32 results (compensated) 1024 x 4096 x 4096 82 us (338) and 300 x 4096
-// x 4096 51 (107).
-// At 1024 x 4096 x 4096 a stage of a 128 x 128 tile takes 1.65 us against 0.43 of MFMAs at 2.4 GHz:
+// kernel, the only one for blocks other than 32 wide); 32-wide blocks, compensated, f16 results, 128 x
+// 4096 x 4096 22 us (45 on the chunk-stream kernel, one pass over the weights per 32 rows) and 1024 x
+// 4096 x 4096 70 us (337); f32 results 78 (337) and 300 x 4096 x 4096 51 (107).
+// A stage of a plain 128 x 128 tile with 32-wide blocks takes 1.65 us against 0.43 of MFMAs at 2.4 GHz:
 // the multiply-adds and the decode are 0.7 us of VALU a SIMD, and the activation reads (1 KiB of LDS
 // per MFMA, as each wave has one 32-channel column) slow the MFMAs further.
 #pragma once
@@ -83,10 +84,11 @@ __device__ __forceinline__ uint32_t tile_decode_pair(uint32_t x, int b)
 }
 
 // SPB: 32-k sub-steps per scaling (1, 2 or 4: the scale block width is a multiple of 32 SPB).
-// COMP > 0: the accumulators are compensated. A plain f32 accumulator adds k / 32 terms; with f32
-// results that chain's rounding would exceed that of the chunk-stream kernel, whose waves sum every
-// sixteenth block and meet in f64. So acc holds the sum of COMP blocks plus the error of the last
-// addition to hi, the running sum (three operations every COMP blocks), and both meet in f64.
+// COMP > 0: the accumulators are compensated. A plain f32 accumulator adds k / 32 terms, a chain whose
+// rounding would exceed that of the chunk-stream kernel, whose waves sum every sixteenth block and meet
+// in f64 (route.hpp: the errors of both and which COMP is taken). So acc holds the sum of COMP blocks
+// plus the error of the last addition to hi, the running sum (four operations every COMP blocks), and
+// both meet in f64.
 template <int MI, int WGN, int KS, int NSMAX, int SPB, int COMP, int OUT>
 __global__ __launch_bounds__(64 * WGN * KS, 2) void w4a16_tile_kernel(F16TileArgs a)
 {
@@ -215,7 +217,8 @@ __global__ __launch_bounds__(64 * WGN * KS, 2) void w4a16_tile_kernel(F16TileArg
         }
     };
 
-    static_assert(COMP == 0 || (SPB == 1 && SUW % COMP == 0), "compensation steps within a stage");
+    static_assert(COMP == 0 || (SPB == 1 && (SUW % COMP == 0 || COMP % SUW == 0)),
+                  "whole compensation steps per stage, or stages per step");
     f32x16 acc[MI], part[MI];
     f32x16 hi[COMP > 0 ? MI : 1];
 #pragma unroll
@@ -368,7 +371,9 @@ __global__ __launch_bounds__(64 * WGN * KS, 2) void w4a16_tile_kernel(F16TileArg
                         c0[r] = 0.f;
                     }
                     // (this adds the block before the sub-step's own)
-                    if (COMP > 0 && q % (COMP > 0 ? COMP : 1) == 0) {
+                    if (COMP > 0 && COMP <= SUW && q % (COMP > 0 ? COMP : 1) == 0) {
+                        compensate(i);
+                    } else if (COMP > SUW && q == 0 && st % (COMP > SUW ? COMP / SUW : 1) == 0) {
                         compensate(i);
                     }
                     // here and not later: sunk towards the end of the loop, as the compiler would,

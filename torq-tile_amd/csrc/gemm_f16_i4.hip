@@ -631,79 +631,37 @@ int device_cu_count()
     return cus > 0 ? cus : 1;
 }
 
-// ---------------------------------------------------------------------------------------------
-// Large-tile kernel (f16_tile.hpp): which tile a shape takes, by the same rule as the int8 tiles.
-// A launch is rounds of 256 tiles, one per CU, of fixed + rate * ceil(k / 128) microseconds; the
-// 4-wave tiles also run two to a CU (a pair of rounds at a cost of its own). Measured on MI355X at
-// k 4096 (32 stages), per round of 256 tiles; pair in parentheses:
-//                     32-wide blocks   64-wide       compensated (f32 results, 32-wide blocks)
-//   128 x 256         110              80
-//   128 x 128         58               50
-//   64 x 128          35 (64)          33 (51)       49 (88)
-//   32 x 64           18 (25)          16 (24)       22 (31)
-// Against the kernels above at 4096 x 4096, 32-wide blocks, f16 results: 12.6 us for 32 rows there
-// (18.7 here), 23.2 for 64 (18.7), 44.3 for 128 (18.8).
-// ---------------------------------------------------------------------------------------------
-struct F16TileShape
-{
-    int bm, bn, threads;
-    float fixed, stage;            // us of one round
-    float pair_fixed, pair_stage;  // us of two
-};
-constexpr int kF16Shapes = 4;
-constexpr F16TileShape kF16Tiles[3][kF16Shapes] = {
-    // 32-wide blocks
-    {{128, 256, 512, 9.f, 3.1f, 18.f, 6.2f}, {128, 128, 512, 6.f, 1.6f, 12.f, 3.2f},
-     {64, 128, 256, 4.5f, .95f, 5.f, 1.85f}, {32, 64, 256, 4.2f, .44f, 5.f, .61f}},
-    // blocks of a multiple of 64
-    {{128, 256, 512, 9.f, 2.2f, 18.f, 4.4f}, {128, 128, 512, 6.f, 1.4f, 12.f, 2.8f},
-     {64, 128, 256, 4.5f, .9f, 5.f, 1.45f}, {32, 64, 256, 4.2f, .38f, 5.f, .58f}},
-    // compensated: the registers of the two larger tiles do not suffice
-    {{0, 0, 0, 0.f, 0.f, 0.f, 0.f}, {0, 0, 0, 0.f, 0.f, 0.f, 0.f},
-     {64, 128, 256, 4.5f, 1.4f, 5.f, 2.6f}, {32, 64, 256, 4.2f, .57f, 5.f, .8f}}};
-
+// Large-tile and few-row kernels (f16_tile.hpp, f16_skinny.hpp); which takes a shape: route.hpp.
 template <int MI, int WGN, int KS, int NS, int SPB, int COMP, int OUT>
 void launch_f16_tile(F16TileArgs t, hipStream_t s)
 {
     constexpr int BM = 32 * MI, BN = 32 * WGN;
     t.tiles_m = (t.M + BM - 1) / BM;
     t.tiles_n = (t.N + BN - 1) / BN;
-    const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;  // (the pick bounds them)
+    const long long tiles = static_cast<long long>(t.tiles_m) * t.tiles_n;  // (the route bounds them)
     t.per_xcd = static_cast<int>((tiles + 7) / 8);
     hipLaunchKernelGGL((w4a16_tile_kernel<MI, WGN, KS, NS, SPB, COMP, OUT>),
                        dim3(8 * static_cast<unsigned>(t.per_xcd)), dim3(64 * WGN * KS), 0, s, t);
 }
 
 template <int SPB, int OUT>
-void launch_f16_tile_shape(int shape, const F16TileArgs &t, hipStream_t s)
+void launch_f16_tile_plain(W4A16Kernel kernel, const F16TileArgs &t, hipStream_t s)
 {
-    switch (shape) {
-    case 0: launch_f16_tile<4, 8, 1, 3, SPB, 0, OUT>(t, s); break;
-    case 1: launch_f16_tile<4, 4, 2, 3, SPB, 0, OUT>(t, s); break;
-    case 2: launch_f16_tile<2, 4, 1, 3, SPB, 0, OUT>(t, s); break;
+    switch (kernel) {
+    case W4A16_TILE_128X256: launch_f16_tile<4, 8, 1, 3, SPB, 0, OUT>(t, s); break;
+    case W4A16_TILE_128X128: launch_f16_tile<4, 4, 2, 3, SPB, 0, OUT>(t, s); break;
+    case W4A16_TILE_64X128: launch_f16_tile<2, 4, 1, 3, SPB, 0, OUT>(t, s); break;
     default: launch_f16_tile<1, 2, 2, 6, SPB, 0, OUT>(t, s); break;
     }
 }
 
-// f32 results with 32-wide blocks. One compensation per block up to k 1536 and per two blocks past
-// it: relative error against 64 bits 4.5e-8 and 4.9e-8 at every k, where the kernels above have
-// 4.4e-8 at k 512, 4.8e-8 at 1024, 5.4e-8 at 2048 and 6.5e-8 at 4096, and plain accumulators
-// 6.2e-8 to 2.7e-7 (64 x 128 tiles at k 4096: 64 us a pair of rounds plain, 88 and 112 compensated).
-inline void launch_f16_tile_comp(int shape, const F16TileArgs &t, hipStream_t s)
+template <int COMP, int OUT>
+void launch_f16_tile_comp(W4A16Kernel kernel, const F16TileArgs &t, hipStream_t s)
 {
-    const bool every = t.K < 1536;
-    if (shape == 2) {
-        if (every) {
-            launch_f16_tile<2, 4, 1, 3, 1, 1, OUT_F32>(t, s);
-        } else {
-            launch_f16_tile<2, 4, 1, 3, 1, 2, OUT_F32>(t, s);
-        }
+    if (kernel == W4A16_TILE_64X128) {
+        launch_f16_tile<2, 4, 1, 3, 1, COMP, OUT>(t, s);
     } else {
-        if (every) {
-            launch_f16_tile<1, 2, 2, 6, 1, 1, OUT_F32>(t, s);
-        } else {
-            launch_f16_tile<1, 2, 2, 6, 1, 2, OUT_F32>(t, s);
-        }
+        launch_f16_tile<1, 2, 2, 6, 1, COMP, OUT>(t, s);
     }
 }
 
@@ -747,29 +705,6 @@ bool tile_layout(const W4A16Args &a)
            a.ldd * kElem < (1 << 23) && (!a.C || a.ldc * kElem < (1 << 23));
 }
 
-// Microseconds of the few-row kernel (f16_skinny.hpp), 0 where it does not apply: a fixed part and
-// the 16-channel strips that one CU streams, more slowly with the activation rows that each strip
-// loads too. At k 4096 and one row: 256 strips 6.5, 512 8.7, 768 10.3, 896 12.1; 1792 strips at k 8192
-// 31; with 16 rows 7.4, 12.3, 13.0, 17.7 and 48.5. More than 16 rows, a group of 16 each, only where
-// the generic kernel is the alternative (26 x 1152 x 11008 in 128-wide blocks 11.7, 36.8 in tiles):
-// the 32-row kernels read the weights once.
-template <int OUT>
-float w4a16_skinny_us(const W4A16Args &a, bool listed)
-{
-    if (a.M > (listed ? 16 : 64) || a.K < 128 || !tile_layout<OUT>(a) ||
-        !w4a16_skinny_scales_exact(a.K, a.bl)) {
-        return 0.f;
-    }
-    const long long strips = static_cast<long long>(a.ntiles) * ((a.M + 15) / 16);
-    if (!grid_fits(a.ntiles, 512)) {
-        return 0.f;
-    }
-    const long long rounds = (strips + kTileCUs - 1) / kTileCUs;
-    const int rows = a.M < 16 ? a.M : 16;
-    return 4.2f + 1.95f / 4096.f * static_cast<float>(rounds) * static_cast<float>(a.K) *
-                      (1.f + 0.0027f * static_cast<float>(rows * rows));
-}
-
 template <int OUT>
 void launch_w4a16_skinny(const W4A16Args &a, bool nan_to_min, hipStream_t s)
 {
@@ -802,61 +737,27 @@ void launch_w4a16_skinny(const W4A16Args &a, bool nan_to_min, hipStream_t s)
     }
 }
 
-// Microseconds of the best tile shape for plain layouts with 16-byte aligned rows and scale blocks
-// of whole 32-k groups, and that shape; 0 where the kernel does not apply (its offsets are 32 bits
-// from a tile's first row). other_us: the chunk-stream or register kernel's, 0 without one.
-struct F16TilePick
-{
-    float us;
-    int variant, shape;
-};
-
 template <int OUT>
-F16TilePick w4a16_tile_pick(const W4A16Args &a, float other_us)
-{
-    F16TilePick best = {0.f, 0, 0};
-    // Under a stage of k and few outputs the generic kernel takes a few microseconds and sums in
-    // the oracle's order.
-    if (a.K < 128 && static_cast<long long>(a.M) * a.N <= 65536) {
-        return best;
-    }
-    // One chunk of k with f32 results: the chunk-stream kernel's sixteen f64-summed blocks are the
-    // more exact (4.5e-8 against 4.7e-8).
-    if ((OUT == OUT_F32 && a.K == kCsK && other_us > 0.f) || !tile_layout<OUT>(a)) {
-        return best;
-    }
-    best.variant = a.bl % 64 == 0 ? 1 : (OUT == OUT_F32 ? 2 : 0);
-    const float stages = static_cast<float>((a.K + 127) / 128);
-    for (int i = best.variant == 2 ? 2 : 0; i < kF16Shapes; ++i) {
-        const F16TileShape &p = kF16Tiles[best.variant][i];
-        const long long tiles = static_cast<long long>((a.M + p.bm - 1) / p.bm) *
-                                ((a.N + p.bn - 1) / p.bn);
-        if (!grid_fits(tiles + 8, p.threads)) {
-            continue;
-        }
-        const long long rounds = (tiles + kTileCUs - 1) / kTileCUs;
-        const float us =
-            static_cast<float>(rounds / 2) * (p.pair_fixed + p.pair_stage * stages) +
-            static_cast<float>(rounds % 2) * (p.fixed + p.stage * stages);
-        if (best.us == 0.f || us < best.us) {
-            best.shape = i;
-            best.us = us;
-        }
-    }
-    return best;
-}
-
-template <int OUT>
-void launch_w4a16_tile(const W4A16Args &a, const F16TilePick &pick, bool nan_to_min,
-                       hipStream_t s)
+void launch_w4a16_tile(const W4A16Args &a, const W4A16Route &r, bool nan_to_min, hipStream_t s)
 {
     const F16TileArgs t = tile_args(a, nan_to_min);
-    if (pick.variant == 1) {
-        launch_f16_tile_shape<2, OUT>(pick.shape, t, s);
-    } else if constexpr (OUT == OUT_F32) {
-        launch_f16_tile_comp(pick.shape, t, s);
-    } else {
-        launch_f16_tile_shape<1, OUT>(pick.shape, t, s);
+    if (a.bl % 64 == 0) {
+        launch_f16_tile_plain<2, OUT>(r.kernel, t, s);
+        return;
+    }
+    switch (r.comp) {
+    case 1: launch_f16_tile_comp<1, OUT>(r.kernel, t, s); break;
+    case 2: launch_f16_tile_comp<2, OUT>(r.kernel, t, s); break;
+    default:
+        if constexpr (OUT == OUT_F16) {  // (f32 results are compensated every one or two blocks)
+            if (r.comp == 4) {
+                launch_f16_tile_comp<4, OUT>(r.kernel, t, s);
+            } else if (r.comp == 8) {
+                launch_f16_tile_comp<8, OUT>(r.kernel, t, s);
+            } else {
+                launch_f16_tile_plain<1, OUT>(r.kernel, t, s);
+            }
+        }
     }
 }
 
@@ -916,30 +817,14 @@ void w4a16_run(size_t m, size_t n, size_t k, size_t bl, const void *A, size_t ld
     // bl 32 and k % 512 == 0: the chunk-stream kernel
     const bool chunk = bl == 32 && k % kCsK == 0 && k >= kCsK && layout_fast && ldsb % 8 == 0 &&
                        aligned16(A) && aligned16(B) && aligned16(scale_b);
-    // Microseconds of the chunk-stream and register kernels, from measurements at one and four
-    // tiles per workgroup: every 32 rows are a pass of their own over the weights.
-    const long long row_groups = static_cast<long long>((m + kMRows - 1) / kMRows);
-    float other_us = 0.f;
-    if (chunk) {
-        const long long wgs = a.ntiles <= kTileCUs ? a.ntiles : (a.ntiles + kCsTiles - 1) / kCsTiles;
-        const long long nwg = a.ntiles > kTileCUs && wgs < kTileCUs ? kTileCUs : wgs;
-        other_us = static_cast<float>((row_groups * nwg + kTileCUs - 1) / kTileCUs) *
-                   (3.5f + 0.97f * static_cast<float>(a.K / kCsK));
-    } else if (fast) {
-        const long long gx = a.ntiles < kTileCUs ? a.ntiles : kTileCUs;
-        const float strip = static_cast<float>(a.ntiles) / static_cast<float>(gx) - 1.f;
-        other_us = static_cast<float>((row_groups * gx + kTileCUs - 1) / kTileCUs) *
-                   (3.5f + static_cast<float>(a.K) * (0.002f + 0.0006f * strip));
-    }
-    const F16TilePick tile = packed ? F16TilePick{0.f, 0, 0} : w4a16_tile_pick<OUT>(a, other_us);
-    const bool listed = other_us > 0.f;
-    const float skinny_us = packed ? 0.f : w4a16_skinny_us<OUT>(a, listed);
-    // (other_us reads about a tenth low against it: 1 x 14336 x 4096 11.3, measured 13.0)
-    if (skinny_us > 0.f && (!listed || skinny_us < 1.1f * other_us) &&
-        (tile.us == 0.f || skinny_us < tile.us)) {
-        launch_w4a16_skinny<OUT>(a, listed, s);
-    } else if (tile.us > 0.f && (!listed || tile.us < other_us)) {
-        launch_w4a16_tile<OUT>(a, tile, listed, s);
+    const W4A16Other other = chunk ? W4A16_CHUNK : (fast ? W4A16_REGISTER : W4A16_GENERIC);
+    const W4A16Route route = packed || !tile_layout<OUT>(a)
+                                 ? W4A16Route{W4A16_OTHER, 0}
+                                 : w4a16_route(m, n, k, bl, OUT == OUT_F32, other);
+    if (route.kernel == W4A16_FEW_ROW) {
+        launch_w4a16_skinny<OUT>(a, other != W4A16_GENERIC, s);
+    } else if (route.kernel != W4A16_OTHER) {
+        launch_w4a16_tile<OUT>(a, route, other != W4A16_GENERIC, s);
     } else if (chunk) {
         const int cus = device_cu_count();  // the current device, per call (no cached state)
         const long long need = (a.ntiles + kCsTiles - 1) / kCsTiles;

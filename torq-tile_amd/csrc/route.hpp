@@ -328,4 +328,173 @@ constexpr bool w4a16_skinny_scales_exact(long long k, long long bl)
     return (k / 32) * (bl / 32) <= 0x100000000ll;
 }
 
+enum W4A16Other  // what takes a shape beside the few-row and the tile kernels
+{
+    W4A16_GENERIC,   // one thread per output
+    W4A16_REGISTER,  // w4a16_mfma_kernel: 32-wide blocks, k % 128 == 0, k <= 4096
+    W4A16_CHUNK      // w4a16_chunk_kernel: 32-wide blocks, k % 512 == 0
+};
+
+enum W4A16Kernel
+{
+    W4A16_OTHER,
+    W4A16_FEW_ROW,
+    W4A16_TILE_128X256,
+    W4A16_TILE_128X128,
+    W4A16_TILE_64X128,
+    W4A16_TILE_32X64
+};
+
+struct W4A16Route
+{
+    W4A16Kernel kernel;
+    int comp;  // tiles: blocks per compensation of the f32 accumulators, 0 for plain ones
+};
+
+// A tile launch is rounds of 256 tiles, one per CU, of fixed + rate * ceil(k / 128) microseconds; the
+// 4-wave tiles also run two to a CU (a pair of rounds at a cost of its own). Measured on MI355X at
+// k 4096 (32 stages), per round of 256 tiles; pair in parentheses:
+//                     32-wide blocks   64-wide    compensated every two 32-wide blocks
+//   128 x 256         110              80
+//   128 x 128         58               50
+//   64 x 128          35 (64)          33 (51)    49 (78)
+//   32 x 64           18 (25)          16 (24)    24 (31)
+struct W4A16Tile
+{
+    W4A16Kernel kernel;
+    int bm, bn, threads;
+    float fixed, stage;            // us of one round
+    float pair_fixed, pair_stage;  // us of two
+};
+constexpr W4A16Tile kW4A16Tiles32[] = {{W4A16_TILE_128X256, 128, 256, 512, 9.f, 3.1f, 18.f, 6.2f},
+                                       {W4A16_TILE_128X128, 128, 128, 512, 6.f, 1.6f, 12.f, 3.2f},
+                                       {W4A16_TILE_64X128, 64, 128, 256, 4.5f, .95f, 5.f, 1.85f},
+                                       {W4A16_TILE_32X64, 32, 64, 256, 4.2f, .44f, 5.f, .61f}};
+constexpr W4A16Tile kW4A16Tiles64[] = {{W4A16_TILE_128X256, 128, 256, 512, 9.f, 2.2f, 18.f, 4.4f},
+                                       {W4A16_TILE_128X128, 128, 128, 512, 6.f, 1.4f, 12.f, 2.8f},
+                                       {W4A16_TILE_64X128, 64, 128, 256, 4.5f, .9f, 5.f, 1.45f},
+                                       {W4A16_TILE_32X64, 32, 64, 256, 4.2f, .38f, 5.f, .58f}};
+// (the registers of the two larger tiles do not suffice for compensated accumulators)
+constexpr W4A16Tile kW4A16TilesComp[] = {{W4A16_TILE_64X128, 64, 128, 256, 4.5f, 1.4f, 5.f, 2.4f},
+                                         {W4A16_TILE_32X64, 32, 64, 256, 4.2f, .6f, 5.f, .8f}};
+
+// Blocks per compensation of the tiles' f32 accumulators with 32-wide blocks. A plain accumulator adds
+// k / 32 terms; the chunk-stream kernel's sixteen waves add k / 512 each and meet in f64, the register
+// kernel's eight k / 256. Relative error against 64 bits, in 1e-8, and microseconds at 1024 x 4096
+// rows and channels:
+//   k                      640    1024   2048   3968   4096   8192   11264
+//   chunk / register       6.6    4.8    5.4    9.6    6.5    8.2    9.3
+//   plain                  8.6   10.6   14.7   20.2   20.5   28.8   33.7    (k 4096: 60 us)
+//   every block            4.5 at every k
+//   every 2 blocks         5.1    5.0    5.0    4.9    4.9    4.9    4.9    (78)
+//   every 4                5.7    5.7    5.6    5.6    5.6    5.5    5.5    (70)
+//   every 8                6.5    6.7    6.7    6.6    6.7    6.6    6.6    (65)
+// f32 results keep within every one or two blocks; f16 results take the widest step whose sums are no
+// further off than those of the kernel that takes the shape otherwise (where that is one thread per
+// output, whose chain is longer than a tile's, plain accumulators).
+constexpr int w4a16_compensation(long long K, bool f32, W4A16Other other)
+{
+    if (f32) {
+        return K < 1536 ? 1 : 2;
+    }
+    if (other == W4A16_CHUNK) {
+        return K < 1536 ? 1 : (K < 3072 ? 2 : (K < 5120 ? 4 : 8));
+    }
+    return other == W4A16_REGISTER ? (K < 640 ? 4 : 8) : 0;
+}
+
+// Microseconds of the chunk-stream and register kernels: every 32 rows are a pass of their own over the
+// weights. The register kernel's, with 16 rows: 4096 x 640 8.2, 1280 x 3840 11.2, 14784 x 256 10.4,
+// 19472 x 896 14.5.
+inline float w4a16_other_us(long long M, long long N, long long K, W4A16Other other)
+{
+    const long long ntiles = ceil_div(N, 16);
+    const long long row_groups = ceil_div(M, 32);
+    const float k = static_cast<float>(K);
+    if (other == W4A16_CHUNK) {
+        const long long wgs = ntiles <= kTileCUs ? ntiles : ceil_div(ntiles, 4);
+        const long long nwg = ntiles > kTileCUs && wgs < kTileCUs ? kTileCUs : wgs;
+        return static_cast<float>(ceil_div(row_groups * nwg, kTileCUs)) *
+               (3.5f + 0.97f * static_cast<float>(K / 512));
+    }
+    const long long gx = ntiles < kTileCUs ? ntiles : kTileCUs;
+    const float strip = static_cast<float>(ntiles) / static_cast<float>(gx) - 1.f;
+    return static_cast<float>(ceil_div(row_groups * gx, kTileCUs)) *
+           (3.5f + k * (0.002f + 0.0006f * strip));
+}
+
+// Microseconds of the few-row kernel, 0 where it does not apply: a fixed part and the 16-channel strips
+// that one CU streams, more slowly with the activation rows that each strip loads too (load blocks for
+// 2, 8 or 16 rows). At k 4096 and one row: 256 strips 6.3, 512 8.7, 688 10.1, 896 12.6; 1792 strips at
+// k 8192 32; with 8 rows 6.3, 688 strips 11.8, 1792 at k 8192 36; with 12 rows 6.9, 14.2 and 41. More
+// than 16 rows, a group of 16 each, only where one thread per output is the alternative (26 x 1152 x
+// 11008 in 128-wide blocks 11.7, 36.8 in tiles): the 32-row kernels read the weights once.
+inline float w4a16_few_row_us(long long M, long long N, long long K, long long bl, W4A16Other other)
+{
+    const long long ntiles = ceil_div(N, 16);
+    if (M > (other == W4A16_GENERIC ? 64 : 16) || K < 128 || !w4a16_skinny_scales_exact(K, bl) ||
+        !grid_fits(ntiles, 512)) {
+        return 0.f;
+    }
+    const float rounds = static_cast<float>(ceil_div(ntiles * ceil_div(M, 16), kTileCUs));
+    const float rows = static_cast<float>(M < 16 ? M : 16);
+    return 4.2f + 1.95f / 4096.f * rounds * static_cast<float>(K) * (1.f + 0.0027f * rows * rows);
+}
+
+// Plain layouts that the tile kernels take (16-byte aligned rows, whole 32-k groups per block).
+inline W4A16Route w4a16_route(long long M, long long N, long long K, long long bl, bool f32,
+                              W4A16Other other)
+{
+    const bool listed = other != W4A16_GENERIC;
+    const float other_us = listed ? w4a16_other_us(M, N, K, other) : 0.f;
+    W4A16Route tile = {W4A16_OTHER, bl % 64 == 0 ? 0 : w4a16_compensation(K, f32, other)};
+    float tile_us = 0.f;
+    // Under a stage of k and few outputs one thread each takes a few microseconds and sums in the
+    // oracle's order; one chunk of k with f32 results: the chunk-stream kernel's sixteen f64-summed
+    // blocks are the more exact (4.5e-8 against 4.7e-8).
+    if (!(K < 128 && M * N <= 65536) && !(f32 && K == 512 && listed)) {
+        const float stages = static_cast<float>(ceil_div(K, 128));
+        // microseconds a stage against those of a compensation every two blocks
+        const float scale = tile.comp == 0 || tile.comp == 2
+                                ? 1.f : (tile.comp == 1 ? 1.4f : (tile.comp == 4 ? 0.89f : 0.82f));
+        auto consider = [&](const W4A16Tile &p) {
+            const long long tiles = ceil_div(M, p.bm) * ceil_div(N, p.bn);
+            if (!grid_fits(tiles + 8, p.threads)) {
+                return;
+            }
+            const long long rounds = ceil_div(tiles, kTileCUs);
+            const float us =
+                static_cast<float>(rounds / 2) * (p.pair_fixed + p.pair_stage * scale * stages) +
+                static_cast<float>(rounds % 2) * (p.fixed + p.stage * scale * stages);
+            if (tile_us == 0.f || us < tile_us) {
+                tile.kernel = p.kernel;
+                tile_us = us;
+            }
+        };
+        if (tile.comp > 0) {
+            for (const W4A16Tile &p : kW4A16TilesComp) {
+                consider(p);
+            }
+        } else {
+            for (int i = 0; i < 4; ++i) {
+                consider(bl % 64 == 0 ? kW4A16Tiles64[i] : kW4A16Tiles32[i]);
+            }
+        }
+    }
+    const float few_us = w4a16_few_row_us(M, N, K, bl, other);
+    // other_us reads low with up to 32 rows, where the weights' stream is most of it (8192 x 8192 19.0,
+    // measured 21; 4096 x 11264 24.8, 25.8; 11008 x 4096 11.3, 13.0). Measured with each layer's weights
+    // from HBM, few rows and the 32-row kernel: 1 x 4096 x 4096 6.3, 11.9; 1 x 14336 x 4096 12.6, 13.8;
+    // 8 x 11008 x 4096 11.8, 13.1; 16 x 8192 x 8192 19.9, 21.1; but 12 x 11008 x 4096 14.2, 13.1; 4 x
+    // 14336 x 4096 14.3, 13.7; 9 x 23200 x 512 10.1, 9.2
+    if (few_us > 0.f && (!listed || few_us < 1.1f * other_us) &&
+        (tile_us == 0.f || few_us < tile_us)) {
+        return {W4A16_FEW_ROW, 0};
+    }
+    if (tile_us > 0.f && (!listed || tile_us < (f32 ? 1.f : 1.08f) * other_us)) {
+        return tile;
+    }
+    return {W4A16_OTHER, 0};
+}
+
 }  // namespace tqt
