@@ -123,16 +123,18 @@ def test_w4a16_tile_infinity(gpu, bl):
     assert np.isfinite(got[rest]).all()
 
 
-@pytest.mark.parametrize("m,n,k,comp", [(256, 4096, 1024, 1), (256, 4096, 2048, 2),
-                                        (256, 4096, 4096, 4), (300, 2050, 8192, 8),
-                                        (1000, 1040, 640, 8)])
-def test_w4a16_tile_f16_sums(gpu, shim, route, m, n, k, comp):
-    """f16 results keep the sums of 32-wide blocks as exact as the chunk-stream and register kernels do
-    (relative error 4.8e-8 at k 1024 to 8.2e-8 at 8192; 9.6e-8 for the register kernel's). C cancels all
-    but the last bits of each sum, so that its error shows beside the 11 bits of the result: at most
-    1e-7 of the sums' rms here, where plain f32 accumulators are off by 1.06e-7 (k 1024), 1.5e-7 (2048),
-    2.0e-7 (4096) and 2.9e-7 (8192). The results' own rounding adds at most 2^-12 of a difference of at
-    most 2^-11 of the sum: 3.5e-8."""
+@pytest.mark.parametrize("m,n,k,comp,bound", [(256, 4096, 1024, 1, 6.8e-8),
+                                              (256, 4096, 2048, 2, 7.2e-8),
+                                              (256, 4096, 4096, 4, 8.0e-8),
+                                              (300, 2050, 8192, 8, 9.5e-8),
+                                              (1000, 1040, 640, 8, 8.3e-8)])
+def test_w4a16_tile_f16_sums(gpu, shim, route, m, n, k, comp, bound):
+    """f16 results keep the sums of 32-wide blocks as exact as the chunk-stream and register kernels do.
+    C cancels all but the last bits of each sum, so that its error shows beside the 11 bits of the
+    result (whose own rounding, at most 2^-12 of a difference of at most 2^-11 of the sum, is part of
+    it): of the sums' rms, the chunk-stream kernel is off by 6.0e-8 at k 1024, 6.5e-8 at 2048, 7.4e-8 at
+    4096 and 9.0e-8 at 8192, plain f32 accumulators by 8.8e-8, 1.1e-7, 1.5e-7 and 2.1e-7. The bounds lie
+    a tenth above the former."""
     route.tqtr_w4a16_route.argtypes = [ctypes.c_longlong] * 4 + [ctypes.c_int] * 2
     got = route.tqtr_w4a16_route(m, n, k, 32, 0, T.W4A16_CHUNK if k % 512 == 0 else T.W4A16_REGISTER)
     assert got % 100 >= T.W4A16_TILE_128X256 and got // 100 == comp
@@ -142,4 +144,4 @@ def test_w4a16_tile_f16_sums(gpu, shim, route, m, n, k, comp):
     out = T.bits_f16(_gr().run_w4a16(shim, d, 0xFBFF, 0x7BFF)).astype(np.float64)
     left = v + T.bits_f16(d["C16"]).astype(np.float64)
     err = np.sqrt(np.mean((out - left) ** 2) / np.mean(v ** 2))
-    assert err <= 1e-7, err
+    assert err <= bound, err

@@ -131,3 +131,16 @@ def test_w4a16_sums(rules, f32, k):
             assert r % 100 < T.W4A16_TILE_128X256 or r // 100 > 0
     assert rules.tqtr_w4a16_route(1024, 4096, 11008, 128, f32, T.W4A16_GENERIC) == \
         T.W4A16_TILE_128X128
+
+
+# (m, n, k, whether the few-row kernel was faster than the 32-row kernels): 32-wide blocks, measured side
+# by side with the weights from HBM
+@pytest.mark.parametrize("m,n,k,few", [
+    (1, 4096, 4096, True), (16, 4096, 4096, True), (1, 14336, 4096, True), (8, 11008, 4096, True),
+    (16, 8192, 8192, True), (8, 28672, 8192, True), (1, 1280, 3840, True), (16, 19472, 896, True),
+    (12, 11008, 4096, False), (4, 14336, 4096, False), (12, 23200, 512, False),
+    (12, 8800, 7168, False),
+])
+def test_w4a16_few_rows(rules, m, n, k, few):
+    other = T.W4A16_CHUNK if k % 512 == 0 else T.W4A16_REGISTER
+    assert (rules.tqtr_w4a16_route(m, n, k, 32, 0, other) == T.W4A16_FEW_ROW) == few

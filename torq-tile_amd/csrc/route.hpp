@@ -418,9 +418,9 @@ inline float w4a16_other_us(long long M, long long N, long long K, W4A16Other ot
                (3.5f + 0.97f * static_cast<float>(K / 512));
     }
     const long long gx = ntiles < kTileCUs ? ntiles : kTileCUs;
-    const float strip = static_cast<float>(ntiles) / static_cast<float>(gx) - 1.f;
+    const float tiles = static_cast<float>(ntiles) / static_cast<float>(gx);  // per workgroup
     return static_cast<float>(ceil_div(row_groups * gx, kTileCUs)) *
-           (3.5f + k * (0.002f + 0.0006f * strip));
+           (3.5f + 1.4f * tiles + k * (0.0008f + 0.0006f * tiles));
 }
 
 // Microseconds of the few-row kernel, 0 where it does not apply: a fixed part and the 16-channel strips
@@ -438,7 +438,9 @@ inline float w4a16_few_row_us(long long M, long long N, long long K, long long b
     }
     const float rounds = static_cast<float>(ceil_div(ntiles * ceil_div(M, 16), kTileCUs));
     const float rows = static_cast<float>(M < 16 ? M : 16);
-    return 4.2f + 1.95f / 4096.f * rounds * static_cast<float>(K) * (1.f + 0.0027f * rows * rows);
+    const float by_rows = M <= 2 ? 1.f : (M <= 8 ? 1.1f + 0.015f * rows : 1.27f + 0.02f * rows);
+    const float round_us = 1.95f / 4096.f * static_cast<float>(K) * by_rows;
+    return 4.2f + rounds * (M > 8 && round_us < 0.95f ? 0.95f : round_us);
 }
 
 // Plain layouts that the tile kernels take (16-byte aligned rows, whole 32-k groups per block).
@@ -487,11 +489,11 @@ inline W4A16Route w4a16_route(long long M, long long N, long long K, long long b
     // from HBM, few rows and the 32-row kernel: 1 x 4096 x 4096 6.3, 11.9; 1 x 14336 x 4096 12.6, 13.8;
     // 8 x 11008 x 4096 11.8, 13.1; 16 x 8192 x 8192 19.9, 21.1; but 12 x 11008 x 4096 14.2, 13.1; 4 x
     // 14336 x 4096 14.3, 13.7; 9 x 23200 x 512 10.1, 9.2
-    if (few_us > 0.f && (!listed || few_us < 1.1f * other_us) &&
+    if (few_us > 0.f && (!listed || few_us < 1.09f * other_us) &&
         (tile_us == 0.f || few_us < tile_us)) {
         return {W4A16_FEW_ROW, 0};
     }
-    if (tile_us > 0.f && (!listed || tile_us < (f32 ? 1.f : 1.08f) * other_us)) {
+    if (tile_us > 0.f && (!listed || tile_us < (f32 || M <= 32 ? 1.f : 1.08f) * other_us)) {
         return tile;
     }
     return {W4A16_OTHER, 0};
