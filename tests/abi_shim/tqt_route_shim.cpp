@@ -37,6 +37,26 @@ int tqtr_w4a16_route(long long m, long long n, long long k, long long bl, int f3
     return r.kernel + 100 * r.comp;
 }
 
+long long tqtr_cf_halo_rows(int OH, int OW, int IH, int SH, int PH, int ext, int pix)
+{
+    return cf_halo_rows(OH, OW, IH, SH, PH, ext, pix);
+}
+
+// The same by a walk over every output row.
+long long tqtr_cf_halo_rows_walk(int OH, int OW, int IH, int SH, int PH, int ext, int pix)
+{
+    const int d = (pix - 1 + OW - 1) / OW;
+    long long most = 0;
+    for (int oh = 0; oh < OH; ++oh) {
+        const int last = oh + d;
+        const long long rows = static_cast<long long>(last / OH) * IH +
+                               cf_clamp_row((last % OH) * SH - PH + ext, IH) -
+                               cf_clamp_row(oh * SH - PH, IH);
+        most = rows > most ? rows : most;
+    }
+    return most;
+}
+
 uint32_t tqtr_scale_block_of(uint32_t kb, uint32_t bdiv)
 {
     return scale_block_of(kb, bdiv, scale_block_inverse(bdiv));

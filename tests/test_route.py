@@ -1,6 +1,8 @@
 """Dispatch rules of the launchers, evaluated on the CPU (torq-tile_amd/csrc/route.hpp)."""
 
 import ctypes
+import random
+import time
 
 import pytest
 
@@ -18,6 +20,8 @@ def rules(route):
     route.tqtr_w8a8_tile.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
     route.tqtr_int8_edge_faster.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
     route.tqtr_w4a16_route.argtypes = [ctypes.c_longlong] * 4 + [ctypes.c_int] * 2
+    for f in (route.tqtr_cf_halo_rows, route.tqtr_cf_halo_rows_walk):
+        f.restype, f.argtypes = ctypes.c_longlong, [ctypes.c_int] * 7
     return route
 
 
@@ -144,3 +148,29 @@ def test_w4a16_sums(rules, f32, k):
 def test_w4a16_few_rows(rules, m, n, k, few):
     other = T.W4A16_CHUNK if k % 512 == 0 else T.W4A16_REGISTER
     assert (rules.tqtr_w4a16_route(m, n, k, 32, 0, other) == T.W4A16_FEW_ROW) == few
+
+
+def test_cf_halo_rows(rules):
+    """The channel-first convolution's halo bound without the walk over the output rows: the same value
+    for any geometry, and no work that grows with the output rows."""
+    rng = random.Random(7)
+    for _ in range(20000):
+        OH, OW, IH = rng.randint(1, 90), rng.randint(1, 90), rng.randint(1, 200)
+        if rng.random() < 0.3:
+            OW = rng.randint(1, 4)
+        SH, PH = rng.choice([0, 1, 1, 2, 3, 7]), rng.choice([0, 1, 2, 3, 9, 60])
+        ext = rng.choice([1, 3, 5, 9, 17, 40])
+        a = (OH, OW, IH, SH, PH, ext, 64)
+        assert rules.tqtr_cf_halo_rows(*a) == rules.tqtr_cf_halo_rows_walk(*a), a
+    wide = (4096, 4096, 4096, 1, 1, 3, 64)
+
+    def best(f):
+        t = []
+        for _ in range(50):
+            t0 = time.perf_counter()
+            f(*wide)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    assert rules.tqtr_cf_halo_rows(*wide) == rules.tqtr_cf_halo_rows_walk(*wide)
+    assert best(rules.tqtr_cf_halo_rows) < 0.5 * best(rules.tqtr_cf_halo_rows_walk)

@@ -42,29 +42,6 @@ struct CfPlan
     int px_rows;  // halo rows at most
 };
 
-// An input row position inside its plane: 0 .. IH.
-__host__ __device__ inline int cf_clamp_row(int row, int IH)
-{
-    return row < 0 ? 0 : (row > IH ? IH : row);
-}
-
-// Halo rows of a tile at most: 64 pixels touch d + 1 consecutive output rows, starting at any row of
-// a plane.
-inline long long cf_halo_rows(const ConvGeom &g)
-{
-    const int d = (kCfPix - 1 + g.OW - 1) / g.OW;
-    long long most = 0;
-    for (int oh = 0; oh < g.OH; ++oh) {
-        const int last = oh + d;
-        const long long rows =
-            static_cast<long long>(last / g.OH) * g.IH +
-            cf_clamp_row((last % g.OH) * g.SH - g.PH + (g.KH - 1) * g.DH + 1, g.IH) -
-            cf_clamp_row(oh * g.SH - g.PH, g.IH);
-        most = rows > most ? rows : most;
-    }
-    return most;
-}
-
 template <int T, int PX>
 __global__ __launch_bounds__(256) void conv_cf_kernel(Int8Args a, CfPlan hp)
 {
@@ -285,7 +262,8 @@ inline bool launch_conv_cf(const Int8Args &a, hipStream_t stream)
     if (a.p0 + a.N > static_cast<long long>(g.ID) * g.OH * g.OW) {
         return false;
     }
-    const long long rows = cf_halo_rows(g);
+    const long long rows =
+        cf_halo_rows(g.OH, g.OW, g.IH, g.SH, g.PH, (g.KH - 1) * g.DH + 1, kCfPix);
     const long long px = rows * g.IW;
     if (rows <= 0 || px > 1024 || (taps == 25 && px > 512)) {
         return false;

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstdint>
+#include <initializer_list>
 
 namespace tqt {
 
@@ -302,6 +303,51 @@ inline bool int8_edge_faster(EdgeForm form, long long M, long long N, long long 
                   0.1f * tail + 0.003f * tiles;
     }
     return tile_us < thread_us;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Channel-first implicit convolution (conv_cf.hpp).
+// ---------------------------------------------------------------------------------------------
+
+// An input row position inside its plane: 0 .. IH.
+constexpr int cf_clamp_row(int row, int IH)
+{
+    return row < 0 ? 0 : (row > IH ? IH : row);
+}
+
+// Input rows that a tile of `pix` consecutive output pixels needs at most: it touches d + 1 output rows,
+// starting at any row oh of a plane. `ext`: input rows between a window's first and one past its last.
+// Rows whose last one lies in the same plane: the difference of two clamped positions, c rows apart, is
+// a trapezoid over the first position oh * SH - PH, so its largest value lies at a row beside an end of
+// the flat part. Rows that reach the next plane: at most d, one by one. (A walk over all output rows
+// took 11 us of host time per call at 4096 of them, also where the call was then refused.)
+inline long long cf_halo_rows(int OH, int OW, int IH, int SH, int PH, int ext, int pix)
+{
+    const int d = (pix - 1 + OW - 1) / OW;
+    long long most = 0;
+    auto take = [&](int oh) {
+        const int last = oh + d;
+        const long long rows = static_cast<long long>(last / OH) * IH +
+                               cf_clamp_row((last % OH) * SH - PH + ext, IH) -
+                               cf_clamp_row(oh * SH - PH, IH);
+        most = rows > most ? rows : most;
+    };
+    const int same = OH - d;  // rows 0 .. same - 1 end in their own plane
+    if (same > 0 && SH > 0) {
+        const long long c = static_cast<long long>(d) * SH + ext;
+        for (long long x : {0ll, IH - c}) {
+            const long long oh = (x + PH) / SH - (x + PH < 0 ? 1 : 0);
+            for (long long r : {oh, oh + 1}) {
+                take(static_cast<int>(r < 0 ? 0 : (r > same - 1 ? same - 1 : r)));
+            }
+        }
+    } else if (same > 0) {
+        take(0);  // every row reads the same input rows
+    }
+    for (int oh = same > 0 ? same : 0; oh < OH; ++oh) {
+        take(oh);
+    }
+    return most;
 }
 
 // ---------------------------------------------------------------------------------------------
