@@ -75,6 +75,13 @@ def test_w4a8_few_rows(rules, m, n, k, ksplit):
     assert rules.tqtr_w4a8_route(m, n, k + 32, 0) != T.W4A8_OTHER
 
 
+def test_w4a8_one_group(rules):
+    """A few outputs of one 32-k group stay with one thread each."""
+    for m, n in ((33, 100), (33, 700), (100, 100)):
+        assert rules.tqtr_w4a8_route(m, n, 32, 0) == T.W4A8_OTHER
+        assert rules.tqtr_w4a8_route(m, n, 64, 0) != T.W4A8_OTHER
+
+
 # (m, n, k, dynamic, packed, whether the few-row kernel was the faster one), measured side by side with
 # the weights from HBM, where the two differ by 8% and more
 @pytest.mark.parametrize("m,n,k,dyn,packed,few", [

@@ -129,7 +129,8 @@ inline bool w4a8_few_row_beats_ksplit(long long M, long long N, long long K)
 }
 
 // Plain operands in the tile kernels' layout. ksplit: the k-split kernel applies (else one thread per
-// output is the alternative, which both others always beat).
+// output is the alternative, which both others beat but for more than 32 rows of one 32-k group: 33 x
+// 700 x 32 4.1 us, in tiles 4.8).
 // The few-row kernel against the tiles, past 8 rows: the activations weigh as much as the weights and
 // each strip reloads them (16 x 28672 x 8192 26.7 us, 24 in tiles; 32 x 28672 x 8192 35, 24).
 // The k-split kernel against the tiles: one pass over the weights per 15 rows, 3.2 us + 0.115 us per
@@ -149,7 +150,7 @@ inline W4A8Route w4a8_route(long long M, long long N, long long K, bool ksplit)
         }
     }
     // (up to 8 rows a pass costs the k-split kernel 0.08 us per 10^6 weights: never in tiles)
-    if (tile_us == 0.f || (ksplit && M <= 8) ||
+    if (tile_us == 0.f || (ksplit && M <= 8) || (M > 32 && K <= 32 && M * N <= 65536) ||
         (ksplit && 3.2f + 0.115e-6f * static_cast<float>(N) * static_cast<float>(K) *
                               static_cast<float>(ceil_div(M, 15)) <= tile_us)) {
         return W4A8_OTHER;
