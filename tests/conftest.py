@@ -31,13 +31,11 @@ def shim():
 @pytest.fixture(scope="session")
 def route():
     """The launchers' dispatch rules (torq-tile_amd/csrc/route.hpp) as a host library."""
-    import ctypes
-
     import tqt_testlib
 
     if not os.path.exists(tqt_testlib.ROUTE_SO):
         pytest.fail("route shim not built: %s" % tqt_testlib.ROUTE_SO)
-    return ctypes.CDLL(tqt_testlib.ROUTE_SO)
+    return tqt_testlib.routes()
 
 
 @pytest.fixture(scope="session")

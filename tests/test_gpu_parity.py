@@ -2,7 +2,7 @@
 
 Shapes: the reference's own test shape lists (test/gemm/test_gemm_i8_i8_rvv.cpp:31-41,
 test/gemm/test_gemm_i8_i4_rvv.cpp:164-179, test/gemm/test_gemm_f16_i4_rvv.cpp:19-49,
-test/conv/test_igemm_i8_i8_rvv.cpp:21-41), the BASELINE.json configurations at full size, and
+test/conv/test_igemm_i8_i8_rvv.cpp:21-41), the benchmark's configurations at full size, and
 extra ragged / aligned shapes that exercise both the MFMA fast paths and the generic paths.
 
 Bar: bit-exact for int32 and int8 outputs and for the W4A8 f32 output (same operation order,
@@ -28,7 +28,7 @@ INT8_FAST_SHAPES = [(64, 256, 512, False), (130, 260, 192, True), (200, 136, 80,
                     # stream kernel with 1, 2, 3 and 5 k-stages of 128 (the column multipliers
                     # after the loop, in the last stage, and the ring shorter than its depth)
                     (64, 256, 128, False), (96, 200, 256, True), (130, 260, 384, False),
-                    (33, 129, 640, True),
+                    (160, 129, 640, True), (33, 129, 640, True),  # (33 rows: the few-row kernel)
                     # 128-row tiles (chosen once they still fill 160 or more CUs), ragged
                     (1200, 2100, 384, True)]
 
@@ -63,7 +63,7 @@ def test_clamp_i32_small_kernel(gpu, m, n, k, with_c):
 
 
 def test_clamp_i32_config1(gpu):
-    """BASELINE cfg 1: A [64,512], B [512,256] uniform in [-128,127], no C, full int32 clamp."""
+    """The benchmark's clamp product: A [64,512], B [512,256] uniform in [-128,127], no C, full int32 clamp."""
     A, B, C = T.gen_clamp(64, 256, 512, seed=42)
     got = _gr().run_clamp(A, B, None, -2**31, 2**31 - 1)
     exp = T.oracle_clamp(A, B, None, -2**31, 2**31 - 1)
@@ -138,7 +138,7 @@ W4A8_FAST_SHAPES = [(1, 160, 256, dict(bias=True)), (4, 100, 512, dict(bias=True
                     (33, 37, 2304, dict(bias=True)), (3, 45, 4352, dict(c=True)),
                     (2, 17, 2048, dict(bias=True)), (31, 33, 512, dict(bias=True, c=True)),
                     (2, 24, 65536, dict()),
-                    # k % 256 != 0 goes to the per-output path
+                    # k % 256 != 0: the few-row kernel and a tile (few rows, and past 32)
                     (15, 48, 384, dict(bias=True)), (33, 37, 640, dict(bias=True))]
 # Decode strip path (m = 1, k = 2048 or 4096): channel counts that leave a wave partly (n % 4)
 # or wholly (n % 16) past n, C, bias, clamps; m = 2-4 at the same k take the MFMA kernel.

@@ -1,10 +1,10 @@
 """GPU parity on seeded random shapes: the W8A8, W4A8 and W4A16 runs through the C ABI against
-the CPU oracle, over shapes drawn so that every kernel path of each type is taken (W8A8: the
-stream kernel for k % 128 == 0, the double-buffered kernel for k % 16 == 0, the per-output kernel
-otherwise; W4A8: the decode strip kernel at m = 1 with k = 2048 / 4096, the MFMA k-split kernel
-for k % 256 == 0, the per-output kernel otherwise; W4A16: the chunk kernel for k % 512 == 0, the
-MFMA kernel for k % 128 == 0, the per-output kernel otherwise), with ragged m and n, C, bias and
-clamps. Same bar as test_gpu_parity: bit-exact for W8A8 and W4A8, within 2 f16 ULP for W4A16."""
+the CPU oracle, over ragged m and n, C, bias and clamps, and k of each class that the dispatch tells
+apart (W8A8: k % 128 == 0, k % 16 == 0, any; W4A8: the decode strip kernel's 2048 and 4096 at m = 1,
+k % 256 == 0, any even k; W4A16: k % 512 == 0, k % 128 == 0, k % 32 == 0); within a class the number of
+rows and channels decides between the few-row, tile and older kernels (torq-tile_amd/csrc/route.hpp).
+Shapes of the W4A8 k-split kernel, which the draws seldom hit, are listed by themselves. Same bar as
+test_gpu_parity: bit-exact for W8A8 and W4A8, within 2 f16 ULP for W4A16."""
 
 import numpy as np
 import pytest
@@ -70,6 +70,21 @@ def test_w4a8_sweep(gpu, i):
                         d["scale_b"])
     np.testing.assert_array_equal(got.view(np.uint32), exp.view(np.uint32),
                                   err_msg="m=%d n=%d k=%d" % (m, n, k))
+
+
+# The k-split kernel's: one chunk of 15 rows and several, one load per lane and several, a ragged last
+# strip of channels, with and without the whole chunk of rows staged
+@pytest.mark.parametrize("m,n,k", [(1, 300, 2816), (2, 515, 2560), (8, 517, 4096), (5, 4000, 5120),
+                                   (17, 100, 256), (24, 1029, 2048), (33, 100, 512), (45, 300, 2048),
+                                   (46, 40, 8192), (61, 515, 1024), (128, 33, 4096)])
+def test_w4a8_ksplit(gpu, m, n, k):
+    assert T.w4a8_route(m, n, k) == T.W4A8_OTHER and k % 256 == 0
+    d = T.gen_w4a8(m, n, k, seed=m + n + k, with_c=bool(m & 1) or m > 40, with_bias=bool(n & 1))
+    cmin, cmax = (-np.inf, np.inf) if m % 2 else (-0.5, 1.0)
+    got = _gr().run_w4a8(d, cmin, cmax)
+    exp = T.oracle_w4a8(d["A"], d["Bp"], d["C"], d["bias"], cmin, cmax, d["scale_a"], d["zp_a"],
+                        d["scale_b"])
+    np.testing.assert_array_equal(got.view(np.uint32), exp.view(np.uint32))
 
 
 def _w4a16_shape(i):

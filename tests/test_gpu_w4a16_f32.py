@@ -114,10 +114,11 @@ def gen(m, n, k, bl, seed, with_c, with_bias=True):
     return d, C, bias
 
 
-# (m, n, k, bl): the strip kernel (k 2048/3072/4096, bl 32), the block kernel (other k % 128,
-# bl 32) and the generic kernel (bl 16, k not a multiple of 128)
+# (m, n, k, bl): the chunk-stream kernel (k % 512 == 0, bl 32), the register kernel (other k % 128,
+# bl 32; the plain call of m 17, as m 5 and 7 are the few-row kernel's) and the generic kernel (bl 16, k
+# not a multiple of 128)
 SHAPES = [(32, 96, 4096, 32), (33, 40, 2048, 32), (7, 50, 3072, 32), (32, 48, 1024, 32),
-          (5, 18, 384, 32), (9, 20, 64, 16), (6, 17, 96, 32), (3, 5, 10, 2),
+          (5, 18, 384, 32), (17, 18, 384, 32), (9, 20, 64, 16), (6, 17, 96, 32), (3, 5, 10, 2),
           (33, 8200, 2048, 32)]
 
 

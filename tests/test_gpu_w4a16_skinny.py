@@ -23,7 +23,7 @@ SHAPES = [
     (7, 515, 11008, 128),
     (1, 8200, 544, 32),      # four waves a workgroup
     (5, 8197, 2304, 64),
-    (16, 8193, 320, 64),
+    (16, 8193, 1088, 64),
     (17, 100, 2880, 96),     # two row groups, the second of one row
     (33, 515, 4224, 64),
     (64, 300, 11008, 128),
@@ -32,6 +32,7 @@ SHAPES = [
 
 @pytest.mark.parametrize("m,n,k,bl", SHAPES)
 def test_w4a16_skinny_f32(gpu, m, n, k, bl):
+    assert T.w4a16_route(m, n, k, bl, 1, k // bl + m % 2)[0] == T.W4A16_FEW_ROW
     d = T.gen_w4a16(m, n, k, bl=bl, seed=m + n + k, with_c=bool(m & 1), with_bias=bool(n & 1))
     lo, hi = (-np.inf, np.inf) if m % 2 else (-3.0, 4.0)
     _check_f32(_run_f32(d, lo, hi, pad_d=n % 3, pad_s=(m % 2)), d, lo, hi)
@@ -39,6 +40,7 @@ def test_w4a16_skinny_f32(gpu, m, n, k, bl):
 
 @pytest.mark.parametrize("m,n,k,bl", SHAPES)
 def test_w4a16_skinny_f16(gpu, shim, m, n, k, bl):
+    assert T.w4a16_route(m, n, k, bl, 0)[0] == T.W4A16_FEW_ROW
     d = T.gen_w4a16(m, n, k, bl=bl, seed=m * 3 + n + k, with_c=bool(m & 1), with_bias=bool(n & 1))
     lo, hi = (-65504.0, 65504.0) if m % 2 else (-2.0, 2.5)
     cmin, cmax = int(T.f16_bits(lo)), int(T.f16_bits(hi))
@@ -52,6 +54,7 @@ def test_w4a16_skinny_infinity(gpu, n):
     """An infinite activation gives infinite results of its sign, NaN where its weight is 0, and
     leaves the other rows alone."""
     m, k = 6, 1024 + 64
+    assert T.w4a16_route(m, n, k, 64, 1)[0] == T.W4A16_FEW_ROW
     d = T.gen_w4a16(m, n, k, bl=64, seed=9)
     d["A16"][2, 100] = 0x7C00
     d["A16"][5, 1000] = 0xFC00

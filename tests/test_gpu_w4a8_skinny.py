@@ -33,6 +33,7 @@ SHAPES = [
 
 @pytest.mark.parametrize("m,n,k", SHAPES)
 def test_w4a8_skinny(gpu, m, n, k):
+    assert T.w4a8_route(m, n, k) == T.W4A8_FEW_ROW
     d = T.gen_w4a8(m, n, k, seed=m + n + k, with_c=bool(m & 1), with_bias=bool(n & 1))
     lo, hi = (-np.inf, np.inf) if m % 2 else (-0.75, 1.25)
     got = _gr().run_w4a8(d, lo, hi)
@@ -46,6 +47,7 @@ def test_w4a8_skinny_extremes(gpu, m):
     """Every product at its largest magnitude over the longest k, and zero points at the int32 limits:
     the sums fit, the correction wraps as in the reference."""
     n, k = 40, 65536
+    assert T.w4a8_route(m, n, k) == T.W4A8_FEW_ROW
     d = T.gen_w4a8(m, n, k, seed=5)
     d["A"][:] = -128
     d["A"][1] = 127
@@ -65,6 +67,7 @@ def test_w4a8_skinny_strides(gpu, m):
 
     g = _gr()
     n, k = 262, 352
+    assert T.w4a8_route(m, n, k) == T.W4A8_FEW_ROW
     lda, ldb, ldc, ldd = k + 48, k + 96, n + 5, n + 3
     d = T.gen_w4a8(m, n, k, seed=11, with_c=True)
     A = np.full((m, lda), 77, np.int8)
@@ -89,6 +92,7 @@ def test_w4a8_skinny_strides(gpu, m):
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("m,n,k", [(10, 131, 2144), (25, 1030, 544)])
 def test_w4a8_skinny_16bit(gpu, shim, bf16, m, n, k):
+    assert T.w4a8_route(m, n, k) == T.W4A8_FEW_ROW
     d = T.gen_w4a8(m, n, k, seed=m + k, with_c=True)
     C16, bias16 = to16(d["C"], bf16), to16(d["bias"], bf16)
     lo, hi = bounds(bf16)

@@ -107,7 +107,8 @@ def check(shim, d, f16, packed, **kw):
 
 
 # (m, n, k): k % 128 == 0 takes the streaming kernel, other k % 16 == 0 the double-buffered
-# kernel, the rest the generic one; m and n not multiples of the 128 tile leave partial tiles
+# kernel (both: the few-row kernel with few rows, which m 1, 33 and the 64 of k 512 are), the rest the
+# generic one; m and n not multiples of the 128 tile leave partial tiles
 SHAPES = [(64, 256, 512), (257, 129, 1024), (1, 128, 4096), (130, 260, 192), (60, 63, 128),
           (3, 8, 11), (60, 63, 127), (33, 70, 96),
           # stream kernel on 128-row tiles, ragged, three k-stages

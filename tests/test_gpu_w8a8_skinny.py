@@ -26,6 +26,7 @@ ROWS_K = [(1, 16), (7, 144), (8, 1024), (9, 1040), (16, 2000), (17, 128), (31, 1
 @pytest.mark.parametrize("m,k", ROWS_K)
 @pytest.mark.parametrize("n", [16, 37, 300])
 def test_w8a8_skinny(gpu, m, k, n):
+    assert T.routes().tqtr_w8a8_few_row(m, n, k, 0, 0)
     d = T.gen_w8a8(m, n, k, seed=m + n + k, with_c=bool(m & 1))
     cmin, cmax = (-128, 127) if m % 2 else (-50, 70)
     got = _gr().run_w8a8(d, cmin, cmax)
@@ -42,6 +43,7 @@ def test_w8a8_skinny_dynamic(gpu, m, k, packed):
 
     g = _gr()
     n = 139
+    assert T.routes().tqtr_w8a8_few_row(m, n, k, 1, bool(packed))
     rng = np.random.default_rng(m * k)
     A = rng.integers(-128, 128, size=(m, k), dtype=np.int64).astype(np.int8)
     B = rng.integers(-127, 128, size=(n, k), dtype=np.int64).astype(np.int8)
@@ -74,6 +76,7 @@ def test_w8a8_skinny_strides(gpu, m):
 
     g = _gr()
     n, k = 70, 1200
+    assert T.routes().tqtr_w8a8_few_row(m, n, k, 0, 0)
     lda, ldb, ldc, ldd = k + 16, k + 48, n + 3, n + 5
     d = T.gen_w8a8(m, n, k, seed=m, with_c=True)
     A = np.full((m, lda), 99, np.int8)

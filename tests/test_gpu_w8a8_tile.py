@@ -1,7 +1,8 @@
 """W8A8 large-tile kernel (outputs of more than one round of 128 x 128 tiles): bit-exact against the
 CPU oracle for 256 x 256 and 128 x 128 tiles, one row and one channel past whole tiles, k of one
-16-byte chunk, of part of a stage and past whole stages, static (C, clamps, shared scale) and per-row
-dynamic (f32, f16) with zero points beyond 16 bits, plain and packed operands, row strides."""
+16-byte chunk, of part of a stage and of more stages than the ring's two, static (C, clamps, shared
+scale) and per-row dynamic (f32, f16) with zero points beyond 16 bits, plain and packed operands, row
+strides. Each test asserts the tile that its call takes."""
 
 import ctypes
 
@@ -59,26 +60,37 @@ def _oracle(d, cmin=-128, cmax=127):
                          int(d.get("qcb", d["B"].shape[0])), d["scale_d"], d["zp_d"])
 
 
-# (m, n, k): 128 x 128 tiles from 257 of them, 256 x 256 where the model has them cheaper
-SHAPES = [(2049, 2049, 16), (2100, 2051, 144), (1153, 4208, 640), (3841, 4097, 272),
-          (4096, 4096, 128), (3900, 8000, 1040)]
+S, B = T.W8A8_TILE_128X128, T.W8A8_TILE_256X256
+
+# (m, n, k, tile)
+SHAPES = [(2049, 2049, 16, S), (2100, 2051, 144, S), (1153, 4208, 656, S), (3841, 4097, 272, S),
+          (3841, 1030, 1280, S), (1540, 8000, 656, B), (3900, 8000, 1040, B)]
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
-def test_w8a8_tile(gpu, m, n, k):
+def _tile(m, n, k, dyn=False):
+    assert not T.routes().tqtr_w8a8_few_row(m, n, k, dyn, 0)
+    return T.routes().tqtr_w8a8_tile(m, n, k, dyn)
+
+
+@pytest.mark.parametrize("m,n,k,tile", SHAPES)
+def test_w8a8_tile(gpu, m, n, k, tile):
+    assert _tile(m, n, k) == tile
     d = _gen(m, n, k, seed=m + k, with_c=k < 700)
     cmin, cmax = (-128, 127) if m % 2 else (-90, 100)
     np.testing.assert_array_equal(_run(d, cmin=cmin, cmax=cmax), _oracle(d, cmin, cmax))
 
 
 @pytest.mark.parametrize("kind", ["w8a8pb", "w8a8p"])
-@pytest.mark.parametrize("m,n,k", [(2100, 2051, 144), (3841, 4097, 272)])
-def test_w8a8_tile_packed(gpu, kind, m, n, k):
+@pytest.mark.parametrize("m,n,k,tile", [(2100, 2051, 144, S), (3841, 4097, 272, S),
+                                        (1153, 4208, 656, S), (1540, 8000, 656, B)])
+def test_w8a8_tile_packed(gpu, kind, m, n, k, tile):
+    assert _tile(m, n, k) == tile
     d = _gen(m, n, k, seed=m + n)
     np.testing.assert_array_equal(_run(d, kind), _oracle(d))
 
 
 def test_w8a8_tile_strides_and_shared_scale(gpu):
+    assert _tile(2177, 2200, 400) == S
     d = _gen(2177, 2200, 400, seed=3)
     d["qcb"] = 1
     np.testing.assert_array_equal(_run(d, lda=432, ldd=2211), _oracle(d))
@@ -86,8 +98,10 @@ def test_w8a8_tile_strides_and_shared_scale(gpu):
 
 @pytest.mark.parametrize("packed", [False, True], ids=["plain", "packed"])
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
-@pytest.mark.parametrize("m,n,k", [(2050, 2052, 208), (3970, 4100, 144)])
-def test_w8a8_tile_dynamic(gpu, shim, f16, packed, m, n, k):
+@pytest.mark.parametrize("m,n,k,tile", [(2050, 2052, 208, S), (3970, 4100, 144, S),
+                                        (3600, 1030, 656, S), (1540, 8000, 1040, B)])
+def test_w8a8_tile_dynamic(gpu, shim, f16, packed, m, n, k, tile):
+    assert _tile(m, n, k, True) == tile
     rng = np.random.default_rng(m + k)
     zp = rng.integers(-128, 128, m).astype(np.int32)
     zp[[5, m - 1]] = [40000, -2 ** 31]

@@ -1,6 +1,5 @@
 """Dispatch rules of the launchers, evaluated on the CPU (torq-tile_amd/csrc/route.hpp)."""
 
-import ctypes
 import random
 import time
 
@@ -11,17 +10,6 @@ import tqt_testlib as T
 
 @pytest.fixture()
 def rules(route):
-    route.tqtr_scale_block_of.restype = ctypes.c_uint32
-    route.tqtr_first_wrong_scale_block.restype = ctypes.c_longlong
-    route.tqtr_first_wrong_scale_block.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
-    route.tqtr_w4a16_skinny_scales_exact.argtypes = [ctypes.c_longlong, ctypes.c_longlong]
-    route.tqtr_w4a8_route.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
-    route.tqtr_w8a8_few_row.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2
-    route.tqtr_w8a8_tile.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
-    route.tqtr_int8_edge_faster.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
-    route.tqtr_w4a16_route.argtypes = [ctypes.c_longlong] * 4 + [ctypes.c_int] * 2
-    for f in (route.tqtr_cf_halo_rows, route.tqtr_cf_halo_rows_walk):
-        f.restype, f.argtypes = ctypes.c_longlong, [ctypes.c_int] * 7
     return route
 
 
@@ -50,7 +38,6 @@ def test_wide_scale_blocks_refused(rules, k, bl):
 
 def test_grid_fits(rules):
     """A grid dimension holds fewer than 2^32 work-items."""
-    rules.tqtr_grid_fits.argtypes = [ctypes.c_longlong, ctypes.c_int]
     assert rules.tqtr_grid_fits((1 << 23) - 1, 512) and not rules.tqtr_grid_fits(1 << 23, 512)
     assert rules.tqtr_grid_fits((1 << 24) - 1, 256) and not rules.tqtr_grid_fits(1 << 24, 256)
 

@@ -29,6 +29,43 @@ EDGE_NK, EDGE_KN_CLAMP, EDGE_KN_REQUANT, EDGE_CONV = range(4)
 W8A8_NO_TILE, W8A8_TILE_128X128, W8A8_TILE_256X256 = range(3)
 GOLDEN_DIR = os.path.join(ROOT, "tests", "golden")
 
+
+def routes():
+    """The dispatch rules as a host library with argument types set."""
+    r = ctypes.CDLL(ROUTE_SO)
+    ll, ci = ctypes.c_longlong, ctypes.c_int
+    r.tqtr_grid_fits.argtypes = [ll, ci]
+    r.tqtr_scale_block_of.restype = ctypes.c_uint32
+    r.tqtr_first_wrong_scale_block.restype = ll
+    r.tqtr_first_wrong_scale_block.argtypes = [ll, ll]
+    r.tqtr_w4a16_skinny_scales_exact.argtypes = [ll, ll]
+    r.tqtr_w4a8_route.argtypes = [ll] * 3 + [ci]
+    r.tqtr_w8a8_few_row.argtypes = [ll] * 3 + [ci] * 2
+    r.tqtr_w8a8_tile.argtypes = [ll] * 3 + [ci]
+    r.tqtr_int8_edge_faster.argtypes = [ci] + [ll] * 4
+    r.tqtr_w4a16_route.argtypes = [ll] * 4 + [ci] * 2
+    for f in (r.tqtr_cf_halo_rows, r.tqtr_cf_halo_rows_walk):
+        f.restype, f.argtypes = ll, [ci] * 7
+    return r
+
+
+def w4a8_route(m, n, k):
+    """The kernel of a plain W4A8 call with aligned rows (m = 1 with k 2048 or 4096 aside: the decode
+    strip kernel)."""
+    return routes().tqtr_w4a8_route(m, n, k, k % 256 == 0 and k <= 65536)
+
+
+def w4a16_route(m, n, k, bl, f32, scale_stride=None):
+    """(kernel, blocks per compensation) of a plain W4A16 call with aligned rows."""
+    ldsb = k // bl if scale_stride is None else scale_stride
+    other = W4A16_GENERIC
+    if bl == 32 and k % 512 == 0 and ldsb % 8 == 0:
+        other = W4A16_CHUNK
+    elif bl == 32 and k % 128 == 0 and k <= 4096 and ldsb % 4 == 0:
+        other = W4A16_REGISTER
+    r = routes().tqtr_w4a16_route(m, n, k, bl, f32, other)
+    return r % 100, r // 100
+
 c_size = ctypes.c_size_t
 c_vp = ctypes.c_void_p
 
