@@ -13,7 +13,8 @@
 // terms; they and the waves' sums are added in f64 and rounded once.
 //
 // What bounds it: the weight stream behind a fixed 4 us (launch and the first loads' latency): 1 x
-// 28672 x 8192 (118 MB) runs at 4.3 TB/s, 31 us. The other kernels' fixed share is larger (they pad
+// 28672 x 8192 (132 MB with the scales) runs at 4.2 TB/s, 32 us; at 1 x 14336 x 4096 the decode and the
+// scaling issue for over half of all cycles beside it. The other kernels' fixed share is larger (they pad
 // to 32 rows and meet all waves at each chunk of k), or they have too few workgroups. Before -> now:
 // 1 x 4096 x 4096 12.0 -> 6.5 us, 1 x 4096 x 14336 31.6 -> 12.0, 1 x 4096 x 11008 in 128-wide blocks
 // 37.3 -> 10.8, 8 x 4096 x 11008 41.7 -> 11.1, 16 x 4096 x 4096 12.3 -> 7.4.

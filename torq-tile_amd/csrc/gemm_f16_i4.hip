@@ -1,7 +1,8 @@
 // gemm_1xnbias_clamp_f16_f16_qsi4c2t (W4A16, block-quantized int4 weights) on gfx950.
 //
-// Many rows, scale blocks other than 32 wide, or k beyond what the kernels below take (plain
-// layouts): the large-tile kernel of f16_tile.hpp.
+// Few rows: the kernel of f16_skinny.hpp; many rows, scale blocks other than 32 wide, or k beyond what
+// the kernels below take: the large-tile kernel of f16_tile.hpp (plain layouts, by the rules of
+// route.hpp).
 //
 // Two MFMA kernels share the math below: w4a16_chunk_kernel (k % 512 == 0: 16 waves per CU walk
 // k in 512-wide chunks streamed through a shared LDS ring; see its own comment) and

@@ -3,10 +3,11 @@
 // m = 1 with k = 2048 or 4096 (plain layouts): the decode strip kernel, wavefront per N-strip
 // with v_dot8_u32_u4 and DPP / lane-swap reductions (described above w4a8_strip_kernel).
 //
-// Many rows, or k not a multiple of 256 (plain layouts, k % 32 == 0): the large-tile kernel of
-// int8_tile.hpp, which reads the weights once per tile of rows instead of once per 15 rows.
+// Other plain layouts with k % 32 == 0: the few-row kernel of int4_skinny.hpp (up to 32 rows), the
+// large-tile kernel of int8_tile.hpp, which reads the weights once per tile of rows instead of once per
+// 15 rows, or the k-split kernel below, by the rules of route.hpp; packed operands take the latter.
 //
-// Few rows (any m in chunks of 15 rows, k % 256 == 0): one workgroup of 8
+// The k-split kernel (any m in chunks of 15 rows, k % 256 == 0): one workgroup of 8
 // wave64s owns a 16-channel weight tile (16 rows of B) for one chunk of up to 15 activation
 // rows; wave w owns one eighth of k.
 //   * Plain weights stream in 128-bit loads shaped 8 rows x 128 bytes per wave instruction
@@ -784,9 +785,9 @@ inline bool tile_layout(const W4A8Args &a)
            aligned16(a.A) && aligned16(a.B) && a.lda < (1 << 22) && a.bstride < (1 << 22);
 }
 
-// Four waves a workgroup where a CU gets more than two strips (16 x 11008 x 4096 6.9, 8.4 with
-// eight) or k leaves eight little to do (1 x 5504 x 1024 3.2, 4.0); eight stream one strip faster
-// (4 x 896 x 13792 5.9, 8.4 with four).
+// Four waves a workgroup where a CU gets more than two strips (16 x 11008 x 4096 6.9 us, 8.4 with
+// eight; weights partly cached) or k leaves eight little to do (1 x 5504 x 1024 3.2, 4.0); eight stream
+// one strip faster (4 x 896 x 13792 5.9, 8.4 with four).
 template <int OUT>
 void launch_w4a8_skinny(const W4A8Args &a, hipStream_t s)
 {

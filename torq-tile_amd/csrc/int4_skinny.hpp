@@ -7,10 +7,11 @@
 // decodes them into the two operands of v_mfma_i32_16x16x64_i8 whose activations are the matching 16
 // byte chunks. The waves meet once, at the end, where their exact int32 partial tiles are added.
 //
-// What bounds it: the weight stream behind a fixed 3.4 us (launch and the first loads' latency); 8 x
-// 28672 x 8192 runs at 5.3 TB/s. Before (k-split kernel, or 32 x 128 tiles where k is no multiple of
-// 256) -> now: 8 x 4096 x 11008 8.1 -> 7.4 us, 9 x 5120 x 12544 15.1 -> 10.7, 16 x 11008 x 4096 12.3
-// -> 6.9, 4 x 896 x 13792 30.8 -> 5.9.
+// What bounds it: the weight stream, with one or two 2 KiB weight blocks in flight per wave (32 KiB a CU
+// at one strip each), behind a fixed 2 to 3 us (launch and the first loads' latency); 8 x 28672 x 8192
+// runs at 5.1 TB/s, 8 x 4096 x 11008 at 3.1. Before (k-split kernel, or 32 x 128 tiles where k is no
+// multiple of 256) -> now, each layer's weights from HBM: 8 x 4096 x 11008 7.9 -> 7.6 us, 9 x 5120 x
+// 13824 15.8 -> 14.6, 16 x 11008 x 4096 13.2 -> 8.8, 4 x 896 x 13824 7.0 -> 5.5, at k 13792 30.8 -> 5.9.
 #pragma once
 
 #include "int8_tile.hpp"

@@ -8,10 +8,11 @@
 // bytes packed when the stage is stored), and stored to LDS as [row][k], rows padded to 144 bytes so
 // that 16 lanes' operand reads touch every bank once. The [k, n] B is turned 4 x 4 bytes at a time.
 //
-// What bounds it: the fetch instructions (per tap byte its bounds and carries). One thread per output,
-// reading both operands byte by byte, took 5430 us for a 2032 x 5169 x 1152 clamp_i32, 110 ms for a
-// 2000 x 4096 x 4100 requantized product and 514 us for a 7 x 7 stride 2 convolution of 3 x 221 x 221
-// pixels to 96 channels; here 62, 88 and 35 us.
+// What bounds it: the fetch instructions (per tap byte its bounds and carries), and for a [k, n] B the
+// turned dword stores (LDS busy 0.42 of the time at 2032 x 5169 x 1152, 0.6 of it bank conflicts). One
+// thread per output, reading both operands byte by byte, took 5430 us for a 2032 x 5169 x 1152
+// clamp_i32, 110 ms for a 2000 x 4096 x 4100 requantized product and 514 us for a 7 x 7 stride 2
+// convolution of 3 x 221 x 221 pixels to 96 channels; here 62, 88 and 35 us.
 #pragma once
 
 namespace tqt {

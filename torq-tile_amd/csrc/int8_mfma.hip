@@ -9,7 +9,7 @@
 //   igemmcf_mx1bias_reqi32toi8_clamp_qai8_qsi8dx_qai8   (B gathered from an NCDHW image)
 // and their packed siblings.
 //
-// Seven kernels, chosen per call:
+// Nine kernels, chosen per call (which of the newer ones takes a shape: route.hpp):
 //   * conv_cf_kernel (conv_cf.hpp; igemmcf with plain weights, 1, 9 or 25 taps, channels a multiple of
 //     16): both operands turned to channel-last in LDS once per workgroup;
 //   * w8a8_tile_kernel (w8a8_tile.hpp; B = [n, k], W8A8 static and dynamic, large outputs): tiles of
@@ -27,8 +27,10 @@
 //   * int8_mfma_kernel (igemmcl, the other 16-byte-aligned shapes, clamp_i32's [k, n] B): 256 threads
 //     (4 wave64s in a 2x2 grid) on a BM x 128 tile, k in steps of 64 bytes through double-buffered
 //     LDS tiles, v_mfma_i32_16x16x64_i8;
+//   * int8_small_clamp_kernel (plain clamp_i32 with few regular tiles): 32 x 32 tiles, k split over four
+//     waves;
 //   * int8_edge_kernel (int8_edge.hpp): plain operands at any alignment, k and channel count;
-//   * int8_generic_kernel: one thread per output for what remains (a few outputs of a short k,
+//   * int8_generic_kernel: one thread per output for what remains (small outputs of a short k,
 //     packed, per-row quantized and channel-first operands that the others refuse).
 // All accumulate exactly in int32 and fuse the epilogue (C, bias, requantization,
 // saturation, clamp) into the store.

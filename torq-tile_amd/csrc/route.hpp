@@ -7,7 +7,9 @@
 
 namespace tqt {
 
-constexpr int kTileCUs = 256;  // compute units of an MI355X
+// Compute units of an MI355X, which the estimates below are for (a device with fewer runs the same
+// kernels, by estimates that fit it less).
+constexpr int kTileCUs = 256;
 
 // Whether `blocks` workgroups of `threads` fit one grid dimension: a launch counts its work-items along
 // a dimension in 32 bits.

@@ -104,8 +104,10 @@ __device__ __forceinline__ void dma_lds16_buf(i32x4 rsrc, int voffset, int8_t *l
 #endif
 }
 
-// The same with a wave-uniform byte offset soffset added (not part of the range check: for loads
-// known to be in range).
+// The same with a wave-uniform byte offset soffset added. The range check covers it: a lane reads zeros
+// where voffset + soffset reaches the resource's num_records (measured with the sum inside the buffer
+// either way: 4608 records and soffset 4096 leave 512 bytes, 512 or no records none), so a resource
+// without records reads zeros whatever the offsets.
 __device__ __forceinline__ void dma_lds16_buf_s(i32x4 rsrc, int voffset, int soffset, int8_t *lds)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
