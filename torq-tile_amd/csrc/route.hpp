@@ -496,14 +496,14 @@ inline float w4a16_few_row_us(long long M, long long N, long long K, long long b
 inline W4A16Route w4a16_route(long long M, long long N, long long K, long long bl, bool f32,
                               W4A16Other other)
 {
-    const bool listed = other != W4A16_GENERIC;
-    const float other_us = listed ? w4a16_other_us(M, N, K, other) : 0.f;
+    const bool other_kernel = other != W4A16_GENERIC;  // a 32-row kernel has the shape otherwise
+    const float other_us = other_kernel ? w4a16_other_us(M, N, K, other) : 0.f;
     W4A16Route tile = {W4A16_OTHER, bl % 64 == 0 ? 0 : w4a16_compensation(K, f32, other)};
     float tile_us = 0.f;
     // Under a stage of k and few outputs one thread each takes a few microseconds and sums in the
     // oracle's order; one chunk of k with f32 results: the chunk-stream kernel's sixteen f64-summed
     // blocks are the more exact (4.5e-8 against 4.7e-8).
-    if (!(K < 128 && M * N <= 65536) && !(f32 && K == 512 && listed)) {
+    if (!(K < 128 && M * N <= 65536) && !(f32 && K == 512 && other_kernel)) {
         const float stages = static_cast<float>(ceil_div(K, 128));
         // microseconds a stage against those of a compensation every two blocks
         const float scale = tile.comp == 0 || tile.comp == 2
@@ -538,11 +538,11 @@ inline W4A16Route w4a16_route(long long M, long long N, long long K, long long b
     // from HBM, few rows and the 32-row kernel: 1 x 4096 x 4096 6.3, 11.9; 1 x 14336 x 4096 12.6, 13.8;
     // 8 x 11008 x 4096 11.8, 13.1; 16 x 8192 x 8192 19.9, 21.1; but 12 x 11008 x 4096 14.2, 13.1; 4 x
     // 14336 x 4096 14.3, 13.7; 9 x 23200 x 512 10.1, 9.2
-    if (few_us > 0.f && (!listed || few_us < 1.09f * other_us) &&
+    if (few_us > 0.f && (!other_kernel || few_us < 1.09f * other_us) &&
         (tile_us == 0.f || few_us < tile_us)) {
         return {W4A16_FEW_ROW, 0};
     }
-    if (tile_us > 0.f && (!listed || tile_us < (f32 || M <= 32 ? 1.f : 1.08f) * other_us)) {
+    if (tile_us > 0.f && (!other_kernel || tile_us < (f32 || M <= 32 ? 1.f : 1.08f) * other_us)) {
         return tile;
     }
     return {W4A16_OTHER, 0};
